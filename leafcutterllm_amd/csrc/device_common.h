@@ -297,16 +297,15 @@ __device__ inline void act16_subblock(const float *v, int64_t t, int d, int sbi,
 // experts fused into the routed launch, in ns slices of sl tokens).  With
 // pslots, routed slot i < nr is pass slot i instead: pass p of expert e
 // (pslots[1 + i] = 256 p + e; nothing when i >= pslots[0]), positions
-// offsets[e] + 32 p onward, at most 32.  Shared launch (shared = 1): slot s
+// offsets[e] + pt p onward, at most pt.  Shared launch (shared = 1): slot s
 // is shared expert s over all T tokens, positions s*T + t.
 struct SlotArgs {
     const int32_t *perm, *counts, *offsets, *touched;
     int E, K, T, shared;
     int nr, S, sbase, ns, sl;
     const int32_t *pslots;  // pass slots (RouterArgs::pass_slots) or null
+    int pt;                 // tokens per matrix-core pass and pass slot: 32 or 64
 };
-
-constexpr int kPassTokens = 32;  // tokens per pass slot
 
 __device__ __forceinline__ bool slot_info(const SlotArgs &sa, int slot, int &e, int &p0, int &n) {
     if (sa.shared) {
@@ -323,12 +322,12 @@ __device__ __forceinline__ bool slot_info(const SlotArgs &sa, int slot, int &e, 
         n = min(sa.sl, sa.T - c * sa.sl);
         return n > 0;
     }
-    if (sa.pslots) {  // one 32-token pass of one expert
+    if (sa.pslots) {  // one pass of one expert
         if (slot >= sa.pslots[0]) return false;
         const int v = sa.pslots[1 + slot], pass = v >> 8;
         e = v & 255;
-        p0 = sa.offsets[e] + kPassTokens * pass;
-        n = min(kPassTokens, sa.counts[e] - kPassTokens * pass);
+        p0 = sa.offsets[e] + sa.pt * pass;
+        n = min(sa.pt, sa.counts[e] - sa.pt * pass);
         return true;
     }
     if (slot >= sa.touched[sa.E]) return false;

@@ -481,6 +481,200 @@ __device__ __forceinline__ void block_pass(g_u8 *const (&wb)[MATS], uint32_t lo,
         step<MATS, SPLIT, LO>(wb, lo, dbo, kb, s_stage0, s_stage1, src, w, acc, wave, lane);
 }
 
+// ---- 64-token passes (one f16 per activation) ------------------------------
+// A wave's MATS x 32 weight rows against two 32-token tiles: each decoded
+// weight operand feeds two MFMAs, and each activation operand read from LDS
+// feeds MATS.  Two partial sums per accumulator (S, then acc += d S) would
+// need 256 registers, so the accumulators hold the sums in units of the
+// current super-block's d instead: with acc in units of d' (the previous
+// scale) a super-block starts with
+//   acc = acc * (d' / d) - (dmin / d) * sum_j m_j V_j
+// and its products sc*q are added to acc by the MFMAs themselves; the result
+// is acc * d of the last super-block.  The rescaling rounds once per
+// super-block and element, as the fma it replaces did.  A super-block with
+// d = 0 keeps d' and decodes with zero scales.
+// Bound: VALU issue beside the MFMAs, and the activation loads.  Per
+// super-block and wave (gate/up) 68 MFMAs against ~530 VALU instructions for
+// 64 tokens, where two 32-token passes issue 68 against ~850; the matrix
+// cores are busy 40% of the launch (26% before).  Without the decode the
+// launch would take 540 of 620 us, without the activation loads 533.
+// Measured (gate/up + down, us, 32-token passes before): config 2 T = 1000
+// 756 + 392 -> 621 + 371, T = 300 286 + 137 -> 264 + 137; config 3 T = 1801
+// 303 + 174 -> 262 + 156, T = 700 149 + 85 -> 138 + 88.
+constexpr int kWide = 64;  // tokens of a wide pass
+constexpr int kSumsOffW = kWide * kTokB<false>;
+constexpr int kStageBytesW = kSumsOffW + kWide * 32;
+__shared__ __attribute__((aligned(1024))) uint8_t s_wide0[kStageBytesW];
+__shared__ __attribute__((aligned(1024))) uint8_t s_wide1[kStageBytesW];
+
+struct WideSrc {
+    g_u8 *tok[16];  // token row bases (wave-uniform): tokens wave + 4 i
+    g_u8 *sums;     // sums array base (wave-uniform)
+    uint32_t soff;  // this lane's byte offset: token 16 wave + lane / 4, 8 bytes
+};
+struct WideRegs {
+    u32x2 tok[8];
+};
+
+__device__ __forceinline__ void wide_load(WideRegs &s, const WideSrc &src, int kb, int half,
+                                          int lane) {
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        s.tok[i] = gload<u32x2>(src.tok[8 * half + i] + (uint32_t)(kb * 1024 + 8 * lane));
+}
+
+__device__ __forceinline__ void wide_store(uint8_t *stage, const WideRegs &s, int half, int wave,
+                                           int lane) {
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        *reinterpret_cast<u32x2 *>(stage + (wave + 32 * half + 4 * i) * kTokB<false> + 8 * lane) =
+            s.tok[i];
+}
+
+__device__ __forceinline__ u32x2 wide_load_sums(const WideSrc &src, int kb) {
+    return gload<u32x2>(src.sums + (src.soff + (uint32_t)kb * 32));
+}
+
+__device__ __forceinline__ void wide_store_sums(uint8_t *stage, u32x2 v, int wave, int lane) {
+    *reinterpret_cast<u32x2 *>(stage + kSumsOffW + wave * 512 + 8 * lane) = v;
+}
+
+// The scale `d` of the coming super-block for accumulators in units of
+// `unit`: d, or `unit` itself when d is zero.  rd = 1 / (the new unit).
+__device__ __forceinline__ float next_unit(float d, float unit, float &rd) {
+    const float u = d != 0.0f ? d : unit;
+    rd = 1.0f / u;
+    return u;
+}
+
+// acc = acc * ratio + t * (sum_j m_j V_j) for NT token tiles
+template <int NT>
+__device__ __forceinline__ void rescale(float16v (&acc)[NT], float ratio, float t,
+                                        const half8 (&amin)[NT], const half8 &mo) {
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        const float16v M = mfma32(amin[j], mo, float16v{});
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[j][i] = __builtin_fmaf(acc[j][i], ratio, t * M[i]);
+    }
+}
+
+// One step of a wide pass (the pipeline of step()): the next super-block's
+// activations pass through registers one token tile at a time (both at once
+// bursts the loads: config 2 gate/up at T = 1000 621 -> 663 us).
+template <int MATS, bool SPLIT, int NT>
+__device__ __forceinline__ void step_wide(g_u8 *const (&wb)[MATS], uint32_t lo,
+                                          const uint32_t (&dbo)[MATS], int kn, const uint8_t *cur,
+                                          uint8_t *nxt, const WideSrc &src, WRaw (&w)[MATS],
+                                          float16v (&acc)[MATS][NT], float (&unit)[MATS], int wave,
+                                          int lane) {
+    const int r = lane & 31, h = lane >> 5;
+    WideRegs act;
+    wide_load(act, src, kn, 0, lane);
+    const u32x2 sums = wide_load_sums(src, kn);
+    __builtin_amdgcn_sched_barrier(0);  // keep the activation loads first
+    Hdr hd[MATS];
+    half8 amin[NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+        amin[j] = *reinterpret_cast<const half8 *>(cur + kSumsOffW + (32 * j + r) * 32 + 16 * h);
+    const _Float16 k0 = h == 0 ? (_Float16)1.0f : (_Float16)0.0f, k1 = (_Float16)1.0f - k0;
+#pragma unroll
+    for (int m = 0; m < MATS; m++) {
+        hd[m] = SPLIT ? unpack_hdr_split(w[m].hdr, w[m].db) : unpack_hdr16(w[m].hdr);
+        w[m].hdr = load_hdr<SPLIT>(wb[m], lo, kn);
+        w[m].db = load_db<SPLIT>(wb[m], dbo[m], kn);
+        float rd;
+        const float u = next_unit(hd[m].d, unit[m], rd);
+        const half8 mo = min_operand(hd[m], h);
+        // lanes of half h hold the mins of sub-blocks 4h .. 4h + 3
+        rescale<NT>(acc[m], unit[m] * rd, -hd[m].dmin * rd, amin, SPLIT ? mo * k0 : mo);
+        if (SPLIT) rescale<NT>(acc[m], 1.0f, -hd[m].dmin2 * rd, amin, mo * k1);
+        unit[m] = u;
+        // d = 0 (d2 in the split layout's second half): zero scales
+        hd[m].sc03 = hd[m].d != 0.0f ? hd[m].sc03 : 0;
+        hd[m].sc47 = (SPLIT ? hd[m].d2 : hd[m].d) != 0.0f ? hd[m].sc47 : 0;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const uint8_t *tokrow = cur + r * kTokB<false>;
+    AUnit a[2][NT];  // [unit parity][token tile], unit u + 1 read ahead
+#pragma unroll
+    for (int j = 0; j < NT; j++) read_a<false>(a[0][j], tokrow + j * 32 * kTokB<false>, 0, h);
+    const uint32_t mg = magic_reg();
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        if (SPLIT && u == 4) {  // sub-blocks 4-7: their own d
+#pragma unroll
+            for (int m = 0; m < MATS; m++) {
+                float rd;
+                const float un = next_unit(hd[m].d2, unit[m], rd);
+                const float ratio = unit[m] * rd;
+#pragma unroll
+                for (int j = 0; j < NT; j++) acc[m][j] *= ratio;
+                unit[m] = un;
+            }
+        }
+        if (NT == 2 && u == 4) {
+            wide_store(nxt, act, 0, wave, lane);
+            wide_load(act, src, kn, 1, lane);
+        }
+        if (u + 1 < 8)
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+                read_a<false>(a[(u + 1) & 1][j], tokrow + j * 32 * kTokB<false>, u + 1, h);
+#pragma unroll
+        for (int m = 0; m < MATS; m++) {
+            half8 blo, bhi;
+            dec_pair(hd[m], u >> 1, w[m].q[u].x, w[m].q[u].y, mg, blo, bhi);
+            w[m].q[u] = load_q<SPLIT>(wb[m], lo, kn, 1 + u, 8 * h);
+#pragma unroll
+            for (int j = 0; j < NT; j++) acc[m][j] = mfma32(a[u & 1][j].h0, blo, acc[m][j]);
+#pragma unroll
+            for (int j = 0; j < NT; j++) acc[m][j] = mfma32(a[u & 1][j].h1, bhi, acc[m][j]);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // bounds the live operands to two units
+    }
+    wide_store(nxt, act, NT - 1, wave, lane);
+    wide_store_sums(nxt, sums, wave, lane);
+    lds_barrier();
+}
+
+// block_pass() for a pass of at most 32 NT tokens; the results are acc * unit
+template <int MATS, bool SPLIT, int NT>
+__device__ __forceinline__ void block_pass_wide(g_u8 *const (&wb)[MATS], uint32_t lo,
+                                                const uint32_t (&dbo)[MATS], int kb0, int kb1,
+                                                const WideSrc &src, float16v (&acc)[MATS][NT],
+                                                float (&unit)[MATS]) {
+    const int lane = threadIdx.x & 63, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int last = kb1 - 1;
+    asm volatile("" : "+s"(kb0));  // see block_pass()
+    WRaw w[MATS];
+    {
+        WideRegs act;
+        wide_load(act, src, kb0, 0, lane);
+#pragma unroll
+        for (int m = 0; m < MATS; m++) load_w<SPLIT>(w[m], wb[m], lo, dbo[m], kb0, h);
+        const u32x2 sums = wide_load_sums(src, kb0);
+        wide_store(s_wide0, act, 0, wave, lane);
+        if (NT == 2) {
+            wide_load(act, src, kb0, 1, lane);
+            wide_store(s_wide0, act, 1, wave, lane);
+        }
+        wide_store_sums(s_wide0, sums, wave, lane);
+    }
+    lds_barrier();
+    int kb = kb0;
+    for (; kb + 2 <= kb1; kb += 2) {
+        step_wide<MATS, SPLIT, NT>(wb, lo, dbo, kb + 1, s_wide0, s_wide1, src, w, acc, unit, wave,
+                               lane);
+        step_wide<MATS, SPLIT, NT>(wb, lo, dbo, min(kb + 2, last), s_wide1, s_wide0, src, w, acc,
+                               unit, wave, lane);
+    }
+    if (kb < kb1)
+        step_wide<MATS, SPLIT, NT>(wb, lo, dbo, kb, s_wide0, s_wide1, src, w, acc, unit, wave, lane);
+}
+
 // ---- 16-token passes -------------------------------------------------------
 // The wave's 32 rows are two 16-row tiles t = 0, 1.  Lane l (r16 = l % 16,
 // c4 = l / 16) loads, for tile t, row 16t + r16's header and the 8 qs bytes
@@ -654,12 +848,29 @@ __device__ __forceinline__ void split16(float v, _Float16 &hi, _Float16 &lo) {
     lo = (_Float16)(v - (float)hi);
 }
 
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ float dpp_f32(float v) {
+    return __uint_as_float(dpp_u32<CTRL, ROW_MASK>(__float_as_uint(v)));
+}
+
+// the sum over each 32-lane half of the wave, in its last lane (register
+// moves only; the row pattern of wave_incl_scan_f64)
+__device__ __forceinline__ float half_wave_sum(float v) {
+    v += dpp_f32<0x111, 0xf>(v);
+    v += dpp_f32<0x112, 0xf>(v);
+    v += dpp_f32<0x114, 0xf>(v);
+    v += dpp_f32<0x118, 0xf>(v);
+    v += dpp_f32<0x142, 0xa>(v);
+    return v;
+}
+
 // token (within the pass) held in C register i by half h
 __device__ __forceinline__ int c_token(int i, int h) { return 8 * (i >> 2) + 4 * h + (i & 3); }
 
 // Each wave of a chain block streams its chain tiles through its own half
 // of one activation stage.
-static_assert(kStageBytes / 8 >= chain_lds_floats(16, 128), "chain tile LDS");
+static_assert(kStageBytes / 8 >= chain_lds_floats(16, 128) && kStageBytesW >= kStageBytes,
+              "chain tile LDS");
 
 // grid (F/128 row blocks, [chain row +] slots, pass groups); block = 4 waves
 // x 32 weight rows.  With ch.tiles, row y = 0 runs the exact router chains
@@ -667,7 +878,9 @@ static_assert(kStageBytes / 8 >= chain_lds_floats(16, 128), "chain tile LDS");
 // LO: x enters as two f16 (hi + lo); otherwise as its hi half alone.  H
 // leaves in the format the down products of the same mode take (with LO
 // its lo halves and the sums of hi + lo, without it sums of hi alone).
-template <bool LO>
+// PT: tokens per pass, 32 or (one f16 per activation, H as f16 pieces) 64; a
+// wide kernel's passes of at most 32 tokens take one token tile.
+template <bool LO, int PT>
 __global__ __launch_bounds__(256, 2) void k_mfma_gateup(
     const uint8_t *__restrict__ gate, const uint8_t *__restrict__ up, int64_t estride,
     const _Float16 *__restrict__ x16, const _Float16 *__restrict__ xs, SlotArgs sa, int d, int F,
@@ -677,8 +890,9 @@ __global__ __launch_bounds__(256, 2) void k_mfma_gateup(
         if (slot == 0) {
             if (blockIdx.z) return;
             const int cw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-            float *lds = reinterpret_cast<float *>(cw < 2 ? s_stage0 : s_stage1) +
-                         (cw & 1) * (kStageBytes / 8);
+            uint8_t *half = PT == kWide ? (cw < 2 ? s_wide0 : s_wide1)
+                                        : (cw < 2 ? s_stage0 : s_stage1);
+            float *lds = reinterpret_cast<float *>(half) + (cw & 1) * (kStageBytes / 8);
             for (int tile = blockIdx.x * kWaves + cw; tile < ch.tiles; tile += gridDim.x * kWaves)
                 chain_tile<8, 128, 1>(ch, tile, lds);
             return;
@@ -700,7 +914,51 @@ __global__ __launch_bounds__(256, 2) void k_mfma_gateup(
     const uint32_t nodb[2] = {0, 0};
     const uint8_t *xb = reinterpret_cast<const uint8_t *>(x16);
     const uint8_t *sb = reinterpret_cast<const uint8_t *>(xs);
-    for (int c = blockIdx.z * kTok; c < n; c += gridDim.z * kTok) {
+    for (int c = blockIdx.z * PT; c < n; c += gridDim.z * PT) {
+        if constexpr (PT == kWide) {
+            WideSrc src;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int tok = slot_token(sa, p0, min(c + wave + 4 * i, n - 1));
+                src.tok[i] = uniform(xb + (int64_t)tok * d * 4);
+            }
+            src.sums = uniform(sb);
+            src.soff = (uint32_t)slot_token(sa, p0, min(c + 16 * wave + (lane >> 2), n - 1)) *
+                           nsb * 4 + 8 * (lane & 3);
+            const auto pass = [&](auto nt) {
+                constexpr int NT = decltype(nt)::value;
+                float16v acc[2][NT] = {};
+                float unit[2] = {1.0f, 1.0f};
+                block_pass_wide<2, false, NT>(wb, r * 16, nodb, 0, NB, src, acc, unit);
+                if (grp0 >= ngrp) return;
+                int fo = f;  // opaque copy: output addresses are formed here (see below)
+                asm volatile("" : "+v"(fo));
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) {
+                        const int q = c + 32 * j + c_token(i, h);
+                        const float v = silu(acc[0][j][i] * unit[0]) * (acc[1][j][i] * unit[1]);
+                        const _Float16 hi = (_Float16)v;
+                        const float part = half_wave_sum((float)hi);
+                        if (q < n) {
+                            const int64_t p = p0 + q;
+                            h16[(p * nkb + (fo >> 8)) * 512 + act16_pos(fo & 255)] = hi;
+                            if (r == 31) {
+                                _Float16 shi, slo;
+                                split16(part, shi, slo);
+                                hs[(p * hsr + grp) * 2] = shi;
+                                hs[(p * hsr + grp) * 2 + 1] = slo;
+                            }
+                        }
+                    }
+            };
+            if (n - c > kTok)
+                pass(std::integral_constant<int, 2>{});
+            else
+                pass(std::integral_constant<int, 1>{});
+            continue;
+        }
         StageSrc src;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
@@ -795,7 +1053,7 @@ __global__ __launch_bounds__(256, 2) void k_mfma_gateup(
 // (the two "matrices" of the pipeline), so each LDS read feeds twice the
 // weight bytes of a 32-row wave.  SPLIT: F is an odd multiple of 128 and the
 // weights are in the split layout (ceil(F / 256) super-blocks per row).
-template <bool SPLIT, bool LO>
+template <bool SPLIT, bool LO, int PT>
 __global__ __launch_bounds__(256, 2) void k_mfma_down(
     const uint8_t *__restrict__ down, int64_t estride, const _Float16 *__restrict__ h16,
     const _Float16 *__restrict__ hs, SlotArgs sa, int d, int F, int ksplit, float *__restrict__ Y,
@@ -833,7 +1091,43 @@ __global__ __launch_bounds__(256, 2) void k_mfma_down(
     float *Yz = Y + (int64_t)bz * split_stride;
     const uint8_t *hb = reinterpret_cast<const uint8_t *>(h16);
     const uint8_t *sb = reinterpret_cast<const uint8_t *>(hs);
-    for (int c = cz * kTok; c < n; c += nz * kTok) {
+    for (int c = cz * PT; c < n; c += nz * PT) {
+        if constexpr (PT == kWide) {
+            WideSrc src;
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                src.tok[i] = uniform(hb + (int64_t)(p0 + min(c + wave + 4 * i, n - 1)) * NB * 1024);
+            src.sums = uniform(sb);
+            src.soff = (uint32_t)(p0 + min(c + 16 * wave + (lane >> 2), n - 1)) * nsb * 4 +
+                       8 * (lane & 3);
+            const uint32_t dbo[2] = {9 * 1024 + 4 * (uint32_t)r,
+                                     9 * 1024 + 4 * (32 + (uint32_t)r) - 32 * 16};
+            const auto pass = [&](auto nt) {
+                constexpr int NT = decltype(nt)::value;
+                float16v acc[2][NT] = {};
+                float unit[2] = {1.0f, 1.0f};
+                block_pass_wide<2, SPLIT, NT>(wb, r * 16, dbo, kb0, kb1, src, acc, unit);
+                if (tile0 >= ntile) return;
+                int rb = tile * 64 + r;  // opaque: output addresses are formed here
+                asm volatile("" : "+v"(rb));
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) {
+                        const int q = c + 32 * j + c_token(i, h);
+                        if (q < n) {
+                            float *yrow = Yz + (int64_t)(p0 + q) * d + rb;
+                            yrow[0] = acc[0][j][i] * unit[0];
+                            yrow[32] = acc[1][j][i] * unit[1];
+                        }
+                    }
+            };
+            if (n - c > kTok)
+                pass(std::integral_constant<int, 2>{});
+            else
+                pass(std::integral_constant<int, 1>{});
+            continue;
+        }
         StageSrc src;
 #pragma unroll
         for (int i = 0; i < 8; i++)
@@ -1600,7 +1894,7 @@ __global__ __launch_bounds__(256) void k_act16(const float *__restrict__ x, int 
 }
 
 SlotArgs dev_slots(const SlotArgsHost &s) {
-    return SlotArgs{s.perm, s.counts, s.offsets, s.touched, s.E, s.K, s.T, s.shared, s.nr, s.S, s.sbase, s.ns, s.sl, s.pslots};
+    return SlotArgs{s.perm, s.counts, s.offsets, s.touched, s.E, s.K, s.T, s.shared, s.nr, s.S, s.sbase, s.ns, s.sl, s.pslots, s.pt};
 }
 
 }  // namespace
@@ -1638,7 +1932,11 @@ hipError_t launch_mfma_gateup(const uint8_t *gate, const uint8_t *up, int64_t es
         c = with_nt(ch, 8);
     }
     if (chunks < 1 || chunks > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(x_lo ? k_mfma_gateup<true> : k_mfma_gateup<false>,
+    const bool wide = sa.pt == kWide;
+    if (wide && (x_lo || hf || !h16)) return hipErrorInvalidValue;
+    auto *kern = wide   ? k_mfma_gateup<false, 64>
+                 : x_lo ? k_mfma_gateup<true, 32> : k_mfma_gateup<false, 32>;
+    hipLaunchKernelGGL(kern,
                        dim3((groups + kWaves - 1) / kWaves, slots + (c.tiles ? 1 : 0), chunks),
                        dim3(256), 0, st, gate, up, estride, x16, xs, dev_slots(sa), d, F, h16, hs,
                        hf, c);
@@ -1681,8 +1979,11 @@ hipError_t launch_mfma_down(const uint8_t *down, int64_t estride, const _Float16
     if (chunks < 1 || ksplit < 1 || (int64_t)chunks * ksplit > 65535) return hipErrorInvalidValue;
     if (F % 128) return hipErrorInvalidValue;
     const dim3 grid((tiles + kWaves - 1) / kWaves, slots, ksplit * chunks);
-    auto *kern = F % 256 ? (h_lo ? k_mfma_down<true, true> : k_mfma_down<true, false>)
-                         : (h_lo ? k_mfma_down<false, true> : k_mfma_down<false, false>);
+    const bool wide = sa.pt == kWide;
+    if (wide && h_lo) return hipErrorInvalidValue;
+    auto *kern = wide  ? (F % 256 ? k_mfma_down<true, false, 64> : k_mfma_down<false, false, 64>)
+                 : h_lo ? (F % 256 ? k_mfma_down<true, true, 32> : k_mfma_down<false, true, 32>)
+                        : (F % 256 ? k_mfma_down<true, false, 32> : k_mfma_down<false, false, 32>);
     hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, down, estride, h16, hs, dev_slots(sa), d, F,
                        ksplit, Y, split_stride);
     return hipGetLastError();

@@ -260,7 +260,7 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
 
 // Exclusive scan of s_off[0..E) (per-expert counts) into offsets by one
 // wave, writing offsets[0..E], touched[] and s_off[E] = total, and with
-// a.pass_slots the pass slots: expert e's ceil(count / 32) passes, in
+// a.pass_slots the pass slots: expert e's ceil(count / pass_tokens) passes, in
 // expert order, after the count of them.
 __device__ void scan_experts(const RouterArgs &a, int *s_off) {
     const int lane = threadIdx.x & 63, E = a.E;
@@ -278,7 +278,7 @@ __device__ void scan_experts(const RouterArgs &a, int *s_off) {
         run += __shfl(incl, 63, 64);
         nt += __popcll(m);
         if (a.pass_slots) {
-            const int passes = (c + kPassTokens - 1) / kPassTokens;
+            const int passes = (c + a.pass_tokens - 1) / a.pass_tokens;
             const int pincl = wave_incl_scan(passes);
             for (int j = 0; j < passes; j++)
                 a.pass_slots[1 + np + pincl - passes + j] = j * 256 + e;

@@ -33,9 +33,10 @@ struct RouterArgs {
     bool x16_lo = true;   // sums of hi + lo (the products take both halves), else of hi
     int32_t *counts, *offsets, *perm, *inv, *touched;
     // pass slots, or null: [0] = their number P, then per slot v < P the
-    // entry pass * 256 + e, the 32-token passes of every touched expert in
-    // expert order (written by the batch dispatch)
+    // entry pass * 256 + e, the passes of pass_tokens tokens of every touched
+    // expert in expert order (written by the batch dispatch)
     int32_t *pass_slots = nullptr;
+    int pass_tokens = 32;
     uint32_t *sync;       // [n_token_groups + 1] zero-initialised counters
     // Fused post-attention RMSNorm (certified fast router only): with xin
     // set, each token block first writes x[t] = rms_norm(xin[t]) * norm_w
@@ -84,9 +85,10 @@ struct SlotArgsHost {
     const int32_t *perm, *counts, *offsets, *touched;
     int E, K, T, shared;
     int nr, S, sbase, ns, sl;
-    // routed slot v < nr is pass slot v (one 32-token pass of one expert)
-    // when set (RouterArgs::pass_slots)
+    // routed slot v < nr is pass slot v (one pass of one expert) when set
+    // (RouterArgs::pass_slots)
     const int32_t *pslots = nullptr;
+    int pt = 32;  // tokens per matrix-core pass: 32, or 64 (one f16 per activation)
 };
 
 // Generic decode path on GGUF-layout tensors (any supported type, any
@@ -123,7 +125,7 @@ hipError_t launch_rpl_down(const uint8_t *down, int64_t estride, const int8_t *h
 // H out in the same format (and/or f32).
 hipError_t launch_act16(const float *x, int T, int d, _Float16 *x16, _Float16 *xs, hipStream_t st,
                         bool lo = true);
-// `chunks` blocks share each slot's 32-token passes (block z takes passes
+// `chunks` blocks share each slot's passes of sa.pt tokens (block z takes passes
 // z, z + chunks, ...), so experts with many tokens spread over the chip.
 hipError_t launch_mfma_gateup(const uint8_t *gate, const uint8_t *up, int64_t estride,
                               const _Float16 *x16, const _Float16 *xs, const SlotArgsHost &sa,

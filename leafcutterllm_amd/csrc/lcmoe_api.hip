@@ -113,11 +113,11 @@ struct lcmoe_handle {
     int64_t t_n[kNumSlots] = {};
 };
 
-// Pass slots a forward of T tokens can need: sum over the touched experts of
-// ceil(count / 32) < T K / 32 + touched.
-static int64_t max_pass_slots(const lcmoe_desc &D, int64_t T) {
+// Pass slots of pt tokens a forward of T tokens can need: sum over the
+// touched experts of ceil(count / pt) < T K / pt + touched.
+static int64_t max_pass_slots(const lcmoe_desc &D, int64_t T, int pt) {
     const int64_t A = T * D.n_expert_used;
-    return (A + 31) / 32 + std::min<int64_t>(D.n_expert, A);
+    return (A + pt - 1) / pt + std::min<int64_t>(D.n_expert, A);
 }
 
 namespace {
@@ -451,7 +451,7 @@ extern "C" lcmoe_status lcmoe_create(const lcmoe_desc *desc, const lcmoe_weights
     if ((st = alloc_n(h, &h->perm, A))) return bail(st);
     if ((st = alloc_n(h, &h->inv, A))) return bail(st);
     if ((st = alloc_n(h, &h->touched, E + 1))) return bail(st);
-    if ((st = alloc_n(h, &h->pass_slots, 1 + max_pass_slots(D, Tm)))) return bail(st);
+    if ((st = alloc_n(h, &h->pass_slots, 1 + max_pass_slots(D, Tm, 32)))) return bail(st);
     const int nsync = router_token_groups((int)Tm, (int)d, (int)E) + 1;
     if ((st = alloc_n(h, &h->sync, nsync))) return bail(st);
     if (hipMemset(h->sync, 0, sizeof(uint32_t) * nsync) != hipSuccess)
@@ -473,11 +473,12 @@ extern "C" void lcmoe_destroy(lcmoe_handle *h) { free_handle(h); }
 // Which product kernels serve an expert family this forward.
 struct Plan {
     bool mfma;
-    bool passes;  // routed slots are pass slots (one 32-token pass each)
+    bool passes;  // routed slots are pass slots (one pass of pt tokens each)
     int slots, ks;
-    int chunks;  // blocks sharing one matrix-core slot's 32-token passes
+    int chunks;  // blocks sharing one matrix-core slot's passes
     int sl, ns;  // fused shared experts: tokens per slot, slots per expert
     int per_slot;  // average tokens per slot
+    int pt;        // tokens per matrix-core pass: 32 or 64
 };
 
 
@@ -510,23 +511,32 @@ static Plan plan_set(lcmoe_handle *h, const ExpertSet &s, bool shared, int T, in
     // passes per block)
     const int64_t per_slot =
         shared ? T : ((int64_t)T * D.n_expert_used + p.slots - 1) / std::max(1, p.slots);
-    p.chunks = p.mfma ? (int)std::min<int64_t>(64, std::max<int64_t>(1, (per_slot + 31) / 32)) : 1;
+    // Passes of 64 tokens (block_pass_wide) where the kernels have them (one
+    // f16 per activation, Q4_K downs) and the touched experts hold more than
+    // one 32-token pass on average: each decoded weight then serves two
+    // token tiles (config 2, us per layer: T = 1000 1208 -> 1044, T = 300 445
+    // -> 422, T = 150 298 -> 282; config 3 T = 1801 550 -> 488).  Below that
+    // average their second tile is mostly padding (config 2 at T = 64, where
+    // no expert needs it, and config 4, 15 tokens on average, gain nothing).
+    p.pt = (s.rpl_dn || s.split_dn) && !h->x_lo && per_slot > 32 ? 64 : 32;
+    p.chunks =
+        p.mfma ? (int)std::min<int64_t>(64, std::max<int64_t>(1, (per_slot + p.pt - 1) / p.pt)) : 1;
     p.per_slot = (int)std::min<int64_t>(per_slot, INT32_MAX);
     // Routed experts averaging more than one pass, and any batch past 32
     // tokens (an expert can then need several passes although the average
     // is under one: config 4 T = 256, 21 of 137 touched experts hold 33-85
-    // tokens): one block per 32-token pass of each touched expert (pass
+    // tokens): one block per pass of pt tokens of each touched expert (pass
     // slots from the dispatch), so busy experts spread over the grid instead
     // of leaving their passes to one block after another (config 4 T = 256:
     // gate/up 570 -> 500 us, down 470 -> 447 us).
     p.passes = p.mfma && !shared && (p.chunks > 1 || T > 32) && h->pass_slots;
     if (p.passes) {
-        p.slots = (int)max_pass_slots(D, T);
+        p.slots = (int)max_pass_slots(D, T, p.pt);
         p.chunks = 1;
     }
     // fused shared experts: slices of the tokens one slot takes (the passes
     // of its chunk blocks, or one row-per-lane pass)
-    p.sl = p.mfma ? 32 * p.chunks : 4;
+    p.sl = p.mfma ? p.pt * p.chunks : 4;
     p.ns = fused ? (T + p.sl - 1) / p.sl : 0;
     const int all = p.slots + fused * p.ns;
     p.ks = p.mfma && s.q8     ? choose_ksplit_q8(s, D.d_model, all * 2 * p.chunks)
@@ -546,7 +556,7 @@ static lcmoe_status run_set(lcmoe_handle *h, ExpertSet &s, bool shared, const fl
     const int A = D.max_tokens * K;  // routed positions; fused shared ones follow
     SlotArgsHost sa{h->perm, h->counts, h->offsets, h->touched, E, K, T, shared ? 1 : 0,
                     pl.slots, fused, fused ? A : INT32_MAX, std::max(1, pl.ns), pl.sl,
-                    pl.passes ? h->pass_slots : nullptr};
+                    pl.passes ? h->pass_slots : nullptr, pl.pt};
     const int slots = pl.slots + fused * pl.ns;
     // H between the products in the form the down kernel reads: f16 pieces
     // for the matrix-core downs, int8 limbs for the row-per-lane ones (Q4_K,
@@ -614,7 +624,7 @@ static lcmoe_status enqueue_forward(lcmoe_handle *h, const float *x, int32_t T, 
     const bool together = Sf > 0 && pr0.chunks == 1;
     const int fused = together ? Sf : 0;
     const Plan pr = together ? plan_set(h, h->routed, false, T, Sf) : pr0;
-    const Plan off{false, false, 0, 1, 1, 4, 0, 0};
+    const Plan off{false, false, 0, 1, 1, 4, 0, 0, 32};
     const Plan pf = Sf > 0 && !together ? plan_set(h, h->routed, false, T, Sf, true) : off;
     const Plan ps = S > 0 && !h->fused ? plan_set(h, h->shared, true, T) : off;
     const bool sep_f = Sf > 0 && !together;
@@ -648,6 +658,7 @@ static lcmoe_status enqueue_forward(lcmoe_handle *h, const float *x, int32_t T, 
     ra.inv = h->inv;
     ra.touched = h->touched;
     ra.pass_slots = pr.passes ? h->pass_slots : nullptr;
+    ra.pass_tokens = pr.pt;
     ra.sync = h->sync;
     // the fast router reads the whole router matrix once per token: past
     // kFastRouterElems multiply-adds per forward the chain router, which
