@@ -10,6 +10,7 @@
 //                  f16 KV cache append (cache/mod.rs:33-63)
 //   k_attn_part /  masked softmax attention (attention.rs:56-115), split
 //   k_attn_combine over 128-position chunks of the context, then merged
+//   k_attn_prefill the same for a prompt's tokens on the matrix cores
 //   k_argmax       greedy sample_top_p (sampler.rs:8-10): max_by(total_cmp),
 //                  the last of equal maxima
 //   k_advance      the cache length after a forward
@@ -26,6 +27,11 @@ namespace lcmoe {
 namespace {
 
 constexpr int kAttnChunk = 128;  // context positions per attention partial
+// Fewest tokens of one sequence that take k_attn_prefill (below, its 32-query
+// tiles are mostly padding; two prompts and two decode steps of the config-5
+// shapes, us, partials + combine against it: 16 tokens 1414 / 1356, 32 tokens
+// 1459 / 1519 before and after on boxes 4% apart).
+constexpr int kPrefillMin = 16;
 
 template <int QT>
 __device__ __forceinline__ void dec8(const uint8_t *row, int64_t k, float (&w)[8]) {
@@ -383,6 +389,248 @@ __global__ __launch_bounds__(256) void k_attn_combine(const float *__restrict__ 
     if (sb < hd / 32) act16_subblock(s_o + 32 * sb, q, H * hd, h * (hd / 32) + sb, x16, xs);
 }
 
+// Prompt attention: a block takes 32 queries of one head (tokens i0 .. i0+31
+// of one sequence) and its eight waves every eighth 32-key tile of the
+// context, each with its own running maximum and sums, merged at the end
+// (the log-sum-exp of k_attn_combine); one launch, no partials in memory.
+// Both products run on v_mfma_f32_32x32x16_f16 (layouts in kern_mfma.hip)
+// with K and V as the cache holds them and q and the probabilities as two
+// f16 (hi + lo, 22 bits) after an exact scaling by a power of two (q's row
+// maximum to 2^14 .. 2^15, probabilities by 2^14, so that lo never runs out
+// of exponents); scores, exponentials and sums are f32:
+//   scores: A = K (keys), B = q, k over the dims, so lane (r, h) gets query
+//           r's scores of keys 8 (i/4) + 4 h + i%4 in register i;
+//   output: A = V^T (row a of tile dt = dim ND a + dt), B = the
+//           probabilities, registers 8 s .. 8 s + 7 being step s's keys as
+//           they lie.
+// A tile that holds an infinite or NaN key or value, also one past a query's
+// position (zero probability times infinity), leaves a result that is not
+// finite: the wave then repeats its tiles in f32, key by key.
+// Bound: latency (a block's waves take ceil(context / 256) tiles each).
+// Measured on the config-5 attention (16 heads x 128), k_attn_part +
+// k_attn_combine before: 500 tokens 117 + 14 -> 22 us, 37 tokens 7 + 5 ->
+// 11 us.  The f32 matrix instruction (v_mfma_f32_32x32x2_f32, an eighth of
+// the rate) in both products took 42 and 19 us; the logits' error against
+// float64 is the same either way and as before (3.7e-5 after 500 tokens,
+// four layers).
+constexpr int kPreWaves = 8;
+
+template <int ND>  // hd = 32 ND
+__global__ __launch_bounds__(64 * kPreWaves, 2) void k_attn_prefill(
+    const float *__restrict__ qr, int T, int seq, const int32_t *__restrict__ lens, int H, int KVH,
+    const _Float16 *__restrict__ kc, const _Float16 *__restrict__ vc, int ctx,
+    float *__restrict__ out, _Float16 *__restrict__ x16, _Float16 *__restrict__ xs) {
+    typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+    typedef _Float16 hv __attribute__((ext_vector_type(ND)));
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef float f16v __attribute__((ext_vector_type(16)));
+    constexpr int HD = 32 * ND, NS = HD / 16, ROW = HD + 4;
+    __shared__ __attribute__((aligned(16))) float s_o[kPreWaves][32][ROW];
+    __shared__ float s_m[kPreWaves][32], s_l[kPreWaves][32];
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int head = blockIdx.y, kvh = head / (H / KVH);
+    // the last queries see the most keys: they go first
+    const int i0 = 32 * ((int)gridDim.x - 1 - (int)blockIdx.x);
+    const int base = lens[seq];                            // cached before this call
+    const int qi = min(i0 + r, T - 1), limit = base + qi;  // query r's token and last key
+    const int nkey = base + min(i0 + 32, T), ntile = (nkey + 31) / 32;
+    const int64_t pstride = (int64_t)KVH * HD;
+    const float *qrow = qr + (int64_t)qi * H * HD + head * HD;
+    const _Float16 *kb = kc + (int64_t)seq * ctx * pstride + kvh * HD;
+    const _Float16 *vb = vc + (int64_t)seq * ctx * pstride + kvh * HD;
+    const float root = sqrtf((float)HD);
+    // key of register i in this lane's half
+    const auto key_of = [&](int i) { return 8 * (i >> 2) + 4 * h + (i & 3); };
+    h8 kv[NS];
+    hv vv[16];
+    // tile kt's rows (clamped to the last key: such keys are masked)
+    const auto load_k = [&](int kt) {
+        const _Float16 *kr = kb + min(32 * kt + r, nkey - 1) * pstride + 8 * h;
+#pragma unroll
+        for (int j = 0; j < NS; j++) kv[j] = *reinterpret_cast<const h8 *>(kr + 16 * j);
+    };
+    const auto load_v = [&](int kt) {
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            vv[i] = *reinterpret_cast<const hv *>(vb + min(32 * kt + key_of(i), nkey - 1) * pstride +
+                                                  ND * r);
+    };
+    if (wave < ntile) load_k(wave);
+    // q, dims 16 j + 8 h .. + 7 of query r, scaled: hi and lo halves
+    h8 qh[NS], ql[NS];
+    float qscale;  // takes the scores back
+    {
+        f4 qv[2 * NS];
+#pragma unroll
+        for (int j = 0; j < NS; j++) {
+            const f4 *qp = reinterpret_cast<const f4 *>(qrow + 16 * j + 8 * h);
+            qv[2 * j] = qp[0];
+            qv[2 * j + 1] = qp[1];
+        }
+        float mx = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 2 * NS; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) mx = fmaxf(mx, fabsf(qv[j][e]));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const int ex = 141 - (int)(__float_as_uint(mx) >> 23);  // mx -> [2^14, 2^15)
+        qscale = __builtin_amdgcn_ldexpf(1.0f, -ex);
+#pragma unroll
+        for (int j = 0; j < NS; j++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float v = __builtin_amdgcn_ldexpf(qv[2 * j + (e >> 2)][e & 3], ex);
+                qh[j][e] = (_Float16)v;
+                ql[j][e] = (_Float16)(v - (float)qh[j][e]);
+            }
+    }
+    f16v O[ND];
+    float m, l;
+    const auto clear = [&] {
+#pragma unroll
+        for (int dt = 0; dt < ND; dt++) O[dt] = f16v{};
+        m = -INFINITY;
+        l = 0.0f;
+    };
+    // scores of a tile -> probabilities, in place; the running maximum moves
+    // on and the sums so far are scaled to it
+    const auto soften = [&](f16v &S, int kt) {
+        float mt = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            S[i] = 32 * kt + key_of(i) <= limit ? S[i] / root : -INFINITY;
+            mt = fmaxf(mt, S[i]);
+        }
+        const float mn = fmaxf(m, fmaxf(mt, __shfl_xor(mt, 32, 64)));
+        const float alpha = m == mn ? 1.0f : expf(m - mn);
+        m = mn;
+        float ps = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            S[i] = S[i] == -INFINITY ? 0.0f : expf(S[i] - mn);
+            ps += S[i];
+        }
+        l = l * alpha + ps;
+#pragma unroll
+        for (int dt = 0; dt < ND; dt++) O[dt] *= alpha;
+    };
+    clear();
+    for (int kt = wave; kt < ntile; kt += kPreWaves) {
+        load_v(kt);  // arrives behind the scores
+        f16v S = f16v{};
+#pragma unroll
+        for (int j = 0; j < NS; j++) S = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[j], ql[j], S, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < NS; j++) S = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[j], qh[j], S, 0, 0, 0);
+        load_k(min(kt + kPreWaves, ntile - 1));
+#pragma unroll
+        for (int i = 0; i < 16; i++) S[i] *= qscale;
+        soften(S, kt);
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            h8 ph, pl;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float v = S[8 * s + e] * 16384.0f;
+                ph[e] = (_Float16)v;
+                pl[e] = (_Float16)(v - (float)ph[e]);
+            }
+#pragma unroll
+            for (int dt = 0; dt < ND; dt++) {
+                h8 a;
+#pragma unroll
+                for (int e = 0; e < 8; e++) a[e] = vv[8 * s + e][dt];
+                O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl, O[dt], 0, 0, 0);
+                O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph, O[dt], 0, 0, 0);
+            }
+        }
+    }
+    bool bad = !(l < INFINITY);
+#pragma unroll
+    for (int dt = 0; dt < ND; dt++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            O[dt][i] *= 1.0f / 16384.0f;
+            bad |= !(fabsf(O[dt][i]) < INFINITY);
+        }
+    if (__ballot(bad)) {
+        clear();
+        float *sp = &s_o[wave][0][0];  // this wave's probabilities, [key][query]
+        for (int kt = wave; kt < ntile; kt += kPreWaves) {
+            f16v S = f16v{};
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const _Float16 *kr = kb + min(32 * kt + key_of(i), nkey - 1) * pstride;
+#pragma unroll 1
+                for (int d = 0; d < HD; d++) S[i] = __builtin_fmaf(qrow[d], (float)kr[d], S[i]);
+            }
+            soften(S, kt);
+#pragma unroll
+            for (int i = 0; i < 16; i++) sp[key_of(i) * ROW + r] = S[i];
+            chain_detail::wave_lds_sync();
+#pragma unroll 1
+            for (int k = 0; k < 32; k++) {
+                const int key = 32 * kt + k;
+                if (key > limit) continue;
+                const float pk = sp[k * ROW + r];
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const hv vk = *reinterpret_cast<const hv *>(vb + key * pstride + ND * key_of(i));
+#pragma unroll
+                    for (int dt = 0; dt < ND; dt++)
+                        O[dt][i] = __builtin_fmaf(pk, (float)vk[dt], O[dt][i]);
+                }
+            }
+            chain_detail::wave_lds_sync();
+        }
+    }
+    l += __shfl_xor(l, 32, 64);
+    if (h == 0) {
+        s_m[wave][r] = m;
+        s_l[wave][r] = l;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; i++) {  // dims ND key_of(i) .. + ND - 1
+        typedef float fv __attribute__((ext_vector_type(ND)));
+        fv v;
+#pragma unroll
+        for (int dt = 0; dt < ND; dt++) v[dt] = O[dt][i];
+        *reinterpret_cast<fv *>(&s_o[wave][r][ND * key_of(i)]) = v;
+    }
+    __syncthreads();
+    // merge: 16 threads per query, HD / 16 dims each; the row also stays in
+    // s_o[0] for the output projection's pieces
+    const int qq = tid >> 4, d0 = (tid & 15) * (HD / 16);
+    float M = -INFINITY, den = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kPreWaves; w++) M = fmaxf(M, s_m[w][qq]);
+    float acc[HD / 16];
+#pragma unroll
+    for (int e = 0; e < HD / 16; e++) acc[e] = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kPreWaves; w++) {
+        const float mw = s_m[w][qq];
+        if (mw != -INFINITY) {
+            const float f = expf(mw - M);
+            den += f * s_l[w][qq];
+#pragma unroll
+            for (int e = 0; e < HD / 16; e++) acc[e] += f * s_o[w][qq][d0 + e];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < HD / 16; e++) {
+        const float v = acc[e] / den;
+        s_o[0][qq][d0 + e] = v;
+        if (i0 + qq < T) out[(int64_t)(i0 + qq) * H * HD + head * HD + d0 + e] = v;
+    }
+    if (!x16) return;
+    __syncthreads();
+    if (tid < 32 * ND && i0 + tid / ND < T)
+        act16_subblock(&s_o[0][tid / ND][32 * (tid % ND)], i0 + tid / ND, H * HD,
+                       head * ND + tid % ND, x16, xs);
+}
+
 // f32::total_cmp order as a signed integer key
 __device__ __forceinline__ int32_t total_key(float v) {
     int32_t b = __float_as_int(v);
@@ -573,6 +821,13 @@ hipError_t launch_attention(const float *qr, int nq, int T, int seq0, const int3
                             _Float16 *xs) {
     if (nq <= 0) return hipSuccess;
     if (x16 && ((H * hd) % 256 || hd % 32 || hd > 256)) return hipErrorInvalidValue;
+    if (nq == T && T >= kPrefillMin && (hd == 32 || hd == 64 || hd == 128)) {  // one sequence
+        const dim3 pg((T + 31) / 32, H), pb(64 * kPreWaves);
+        auto *kern = hd == 32 ? k_attn_prefill<1> : hd == 64 ? k_attn_prefill<2> : k_attn_prefill<4>;
+        hipLaunchKernelGGL(kern, pg, pb, 0, st, qr, T, seq0, lens, H, KVH, kc, vc, ctx, out, x16,
+                           xs);
+        return hipGetLastError();
+    }
     const int chunks = (ctx + kAttnChunk - 1) / kAttnChunk;
     const dim3 grid(nq, H, chunks);
     if (hd <= 64)
