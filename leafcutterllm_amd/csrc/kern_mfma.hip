@@ -10,9 +10,9 @@
 // so every per-row quantity (super-block scales d / dmin, 6-bit sub-block
 // scales and mins) is lane-local.
 //
-// Exact operands: B = sc_j * q (6-bit * 4-bit integers, exact in f16), built
-// from the nibbles as the f16 bit pattern 0x6400 | q = 1024 + q and one
-// packed-f16 fma (1024+q)*sc - 1024*sc.  Activations enter as one f16 per
+// Exact operands: B = sc_j * q * 2^-14 (6-bit * 4-bit integers, exact in
+// f16), built from the nibbles as f16 subnormals and one packed-f16 multiply
+// (dec_pair).  Activations enter as one f16 per
 // element (LO = false, the default mode) or as two f16 halves hi + lo
 // (lo = v - hi rounded again, about 22 significant bits).  Per
 // super-block
@@ -98,8 +98,10 @@ constexpr uint32_t kSel11 = 0x04010401u;
 constexpr uint32_t kSel22 = 0x04020402u;
 constexpr uint32_t kSel33 = 0x04030403u;
 
-// Per-row super-block header (d, dmin, 12 packed scale bytes) unpacked;
-// d2, dmin2: the scales of sub-blocks 4-7 in the split layout.
+constexpr float kDecUnit = 16384.0f;  // dec_pair's operands are sc*q / kDecUnit
+
+// Per-row super-block header (d, dmin, 12 packed scale bytes) unpacked, d
+// times kDecUnit; d2, dmin2: the scales of sub-blocks 4-7 in the split layout.
 struct Hdr {
     uint32_t sc03, sc47, m03, m47;
     float d, dmin, d2, dmin2;
@@ -113,7 +115,7 @@ __device__ __forceinline__ Hdr unpack_hdr16(u32x4 h) {
     s.m03 = h.z & 0x3F3F3F3Fu;
     s.sc47 = (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
     s.m47 = ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u);
-    s.d = dh2f(h.x & 0xffff);
+    s.d = dh2f(h.x & 0xffff) * kDecUnit;
     s.dmin = dh2f(h.x >> 16);
     s.d2 = s.d;
     s.dmin2 = s.dmin;
@@ -122,54 +124,45 @@ __device__ __forceinline__ Hdr unpack_hdr16(u32x4 h) {
 
 __device__ __forceinline__ Hdr unpack_hdr_split(u32x4 h, uint32_t db) {
     Hdr s = unpack_hdr16(h);
-    s.d2 = dh2f(db & 0xffff);
+    s.d2 = dh2f(db & 0xffff) * kDecUnit;
     s.dmin2 = dh2f(db >> 16);
     return s;
 }
 
-// Scales of pair p: s2 = (sc_2p, sc_2p+1 / 16) and c2 = -1024 * s2.  The
-// low-nibble sub-block 2p decodes as (1024 + q) * sc_2p - 1024 * sc_2p; the
-// high-nibble sub-block 2p+1 is decoded unshifted, from the byte 16q, as
-// (1024 + 16q) * (sc / 16) - 64 * sc.  Every step is exact in f16 (the fmas
-// round only their final, integer results <= 945).
-__device__ __forceinline__ void pair_scales(const Hdr &s, int p, half2v &s2, half2v &c2) {
+// Weight operands are sc*q scaled by 2^-14 (Hdr::d carries 2^14 back): a
+// nibble left in the low bits of a 16-bit half is the f16 subnormal
+// q * 2^-24, one and, and one packed multiply by sc * 2^10 makes it the
+// normal number sc*q * 2^-14 -- exact: an integer of at most 10 bits times a
+// power of two.  The high nibbles stay in place as 16 q * 2^-24 and take
+// sc * 2^6.  (An and-or with the exponent of 1024 and a packed fma that
+// takes 1024 sc away again decode as exactly, the bits of every result the
+// same; both are three-operand instructions, and an and issues at twice an
+// and-or's rate beside another wave's VALU work.  Measured with them before:
+// config 3 T = 1801 gate/up 262 -> 249 us, down 156 -> 150; config 2
+// T = 1000 621 -> 605; config 5's layer at T = 16, two f16 per activation,
+// 96.3 -> 94.1 us per call; config 2 T = 64 within 1%.)
+
+// Scales of pair p: (sc_2p * 2^10, sc_2p+1 * 2^6), exact in f16
+__device__ __forceinline__ half2v pair_scales(const Hdr &s, int p) {
     const uint32_t w = p < 2 ? s.sc03 : s.sc47;
     const half2v mag = magic2(w, (p & 1) ? kSel23 : kSel01);  // 1024 + sc
-    s2 = __builtin_elementwise_fma(mag, half2v{(_Float16)1.0f, (_Float16)0.0625f},
-                                   half2v{(_Float16)-1024.0f, (_Float16)-64.0f});
-    c2 = s2 * half2v{(_Float16)-1024.0f, (_Float16)-1024.0f};
+    return (mag - half2v{(_Float16)1024.0f, (_Float16)1024.0f}) *
+           half2v{(_Float16)1024.0f, (_Float16)64.0f};
 }
 
-// Two f16 magic values from the nibbles of bytes 0 and 2 of w, one and-or:
-// the low nibbles (mask 0x000F000F) as 1024 + q, the high ones (0x00F000F0)
-// as 1024 + 16 q
-// mg: kMagicH held in a vector register (magic_reg()), so that the and-or
-// takes the mask as its one constant operand
-constexpr uint32_t kMagicH = 0x64006400u;
-__device__ __forceinline__ half2v nib2(uint32_t w, uint32_t mask, uint32_t mg) {
-    return as_h2((w & mask) | mg);
-}
-__device__ __forceinline__ uint32_t magic_reg() {
-    uint32_t mg = kMagicH;
-    asm volatile("" : "+v"(mg));
-    return mg;
-}
-
-// B operands (sc*q, 8 columns each) of pair p's two sub-blocks from one
-// lane's 8 qs bytes w0, w1 (bytes j = columns j), in the activation format's
-// column order (act16_pos): bytes 0, 2, 1, 3, 4, 6, 5, 7.  Per pair of
-// weights one and-or and one packed fma; the shifted words w >> 8 bring
-// bytes 1 and 3 down to the places of 0 and 2.
+// B operands (sc*q * 2^-14, 8 columns each) of pair p's two sub-blocks from
+// one lane's 8 qs bytes w0, w1 (bytes j = columns j), in the activation
+// format's column order (act16_pos): bytes 0, 2, 1, 3, 4, 6, 5, 7.  The
+// shifted words w >> 8 bring bytes 1 and 3 down to the places of 0 and 2.
 __device__ __forceinline__ void dec_pair(const Hdr &s, int p, uint32_t w0, uint32_t w1,
-                                         uint32_t mg, half8 &blo, half8 &bhi) {
-    half2v s2, c2;
-    pair_scales(s, p, s2, c2);
+                                         half8 &blo, half8 &bhi) {
+    const half2v s2 = pair_scales(s, p);
     const uint32_t w[4] = {w0, w0 >> 8, w1, w1 >> 8};
-    const half2v sl{s2[0], s2[0]}, cl{c2[0], c2[0]}, sh{s2[1], s2[1]}, ch{c2[1], c2[1]};
+    const half2v sl{s2[0], s2[0]}, sh{s2[1], s2[1]};
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const half2v a = __builtin_elementwise_fma(nib2(w[i], 0x000F000Fu, mg), sl, cl);
-        const half2v b = __builtin_elementwise_fma(nib2(w[i], 0x00F000F0u, mg), sh, ch);
+        const half2v a = as_h2(w[i] & 0x000F000Fu) * sl;
+        const half2v b = as_h2(w[i] & 0x00F000F0u) * sh;
         blo[2 * i] = a[0];
         blo[2 * i + 1] = a[1];
         bhi[2 * i] = b[0];
@@ -334,12 +327,12 @@ __device__ __forceinline__ void read_a(AUnit &a, const uint8_t *tokrow, int u, i
 // 2p+1 (high nibbles), four MFMAs per matrix (two without lo halves).
 template <int MATS, bool LO = true>
 __device__ __forceinline__ void unit_mfma(const WRaw (&w)[MATS], const Hdr (&hd)[MATS], int u,
-                                          const AUnit &a, uint32_t mg, float16v (&S)[MATS]) {
+                                          const AUnit &a, float16v (&S)[MATS]) {
     const int p = u >> 1;
 #pragma unroll
     for (int m = 0; m < MATS; m++) {
         half8 blo, bhi;
-        dec_pair(hd[m], p, w[m].q[u].x, w[m].q[u].y, mg, blo, bhi);
+        dec_pair(hd[m], p, w[m].q[u].x, w[m].q[u].y, blo, bhi);
         S[m] = mfma32(a.h0, blo, S[m]);
         if constexpr (LO) S[m] = mfma32(a.l0, blo, S[m]);
         S[m] = mfma32(a.h1, bhi, S[m]);
@@ -421,11 +414,10 @@ __device__ __forceinline__ void step(g_u8 *const (&wb)[MATS], uint32_t lo,
     const half8 *aminp = reinterpret_cast<const half8 *>(cur + kSumsOffT<LO> + r * 32 + 16 * h);
     AUnit a[2];  // unit u's operands, and unit u+1's read ahead
     read_a<LO>(a[0], tokrow, 0, h);
-    const uint32_t mg = magic_reg();
 #pragma unroll
     for (int u = 0; u < 8; u++) {
         if (u + 1 < 8) read_a<LO>(a[(u + 1) & 1], tokrow, u + 1, h);
-        unit_mfma<MATS, LO>(w, hd, u, a[u & 1], mg, S);
+        unit_mfma<MATS, LO>(w, hd, u, a[u & 1], S);
 #pragma unroll
         for (int m = 0; m < MATS; m++) w[m].q[u] = load_q<SPLIT>(wb[m], lo, kn, 1 + u, 8 * h);
         if (SPLIT && u == 3) {  // sub-blocks 0-3 done: their own d
@@ -600,7 +592,6 @@ __device__ __forceinline__ void step_wide(g_u8 *const (&wb)[MATS], uint32_t lo,
     AUnit a[2][NT];  // [unit parity][token tile], unit u + 1 read ahead
 #pragma unroll
     for (int j = 0; j < NT; j++) read_a<false>(a[0][j], tokrow + j * 32 * kTokB<false>, 0, h);
-    const uint32_t mg = magic_reg();
 #pragma unroll
     for (int u = 0; u < 8; u++) {
         if (SPLIT && u == 4) {  // sub-blocks 4-7: their own d
@@ -625,7 +616,7 @@ __device__ __forceinline__ void step_wide(g_u8 *const (&wb)[MATS], uint32_t lo,
 #pragma unroll
         for (int m = 0; m < MATS; m++) {
             half8 blo, bhi;
-            dec_pair(hd[m], u >> 1, w[m].q[u].x, w[m].q[u].y, mg, blo, bhi);
+            dec_pair(hd[m], u >> 1, w[m].q[u].x, w[m].q[u].y, blo, bhi);
             w[m].q[u] = load_q<SPLIT>(wb[m], lo, kn, 1 + u, 8 * h);
 #pragma unroll
             for (int j = 0; j < NT; j++) acc[m][j] = mfma32(a[u & 1][j].h0, blo, acc[m][j]);
@@ -772,7 +763,6 @@ __device__ __forceinline__ void step16(g_u8 *const (&wb)[MATS], uint32_t lo,
     const half4 *aminp = reinterpret_cast<const half4 *>(cur + kSumsOffT<LO> + r16 * 32 + 8 * c4);
     AUnit a[2];  // pair p's operands, and pair p+1's read ahead
     read_a16<LO>(a[0], tokrow, 0, c4);
-    const uint32_t mg = magic_reg();
 #pragma unroll
     for (int p = 0; p < 4; p++) {
         if (p + 1 < 4) read_a16<LO>(a[(p + 1) & 1], tokrow, p + 1, c4);
@@ -782,7 +772,7 @@ __device__ __forceinline__ void step16(g_u8 *const (&wb)[MATS], uint32_t lo,
 #pragma unroll
             for (int t = 0; t < 2; t++) {
                 half8 blo, bhi;
-                dec_pair(hd[m][t], p, w[m].q[p][t].x, w[m].q[p][t].y, mg, blo, bhi);
+                dec_pair(hd[m][t], p, w[m].q[p][t].x, w[m].q[p][t].y, blo, bhi);
                 w[m].q[p][t] = load_q16<SPLIT>(wb[m], lo, kn, p, t, c4);
                 S[m][t] = mfma16(h0, blo, S[m][t]);
                 if constexpr (LO) S[m][t] = mfma16(l0, blo, S[m][t]);
