@@ -44,6 +44,14 @@ __device__ __forceinline__ void store_agent(int32_t *p, int32_t v) {
 __device__ __forceinline__ int32_t load_agent(const int32_t *p) {
     return __hip_atomic_load(const_cast<int32_t *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ void store_agent_u64(uint64_t *p, uint64_t v) {
+    __hip_atomic_store(reinterpret_cast<unsigned long long *>(p), (unsigned long long)v,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t load_agent_u64(const uint64_t *p) {
+    return __hip_atomic_load(reinterpret_cast<unsigned long long *>(const_cast<uint64_t *>(p)),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // Routing weights of token t from its scores s_z (sigmoid scores s_s for the
 // group router) and its selection sel[0..K), in slot order, by one wave: the
@@ -369,6 +377,64 @@ __device__ void dispatch_block(const RouterArgs &a, int (*s_cw)[kMaxE], int *s_o
     }
 }
 
+// The same dispatch of at most 64 GMAX assignments by one wave, without the
+// block's barriers and LDS counters: assignment 64 g + l sits in lane l, the
+// ballots of its expert's eight bits give every lane both its own matches
+// (rank) and, reading the lane number as an expert, that expert's count.
+// s_off: E + 1 counts in LDS, then offsets.
+constexpr int kDispGroups = 4;
+
+__device__ void dispatch_wave(const RouterArgs &a, int *s_off) {
+    const int lane = threadIdx.x & 63, A = a.T * a.K, E = a.E;
+    const uint64_t below = (1ull << lane) - 1ull;
+    int ev[kDispGroups];
+#pragma unroll
+    for (int g = 0; g < kDispGroups; g++)
+        ev[g] = 64 * g + lane < A ? load_agent(a.topk_idx + 64 * g + lane) : -1;
+    int cnt[4] = {0, 0, 0, 0};      // expert 64 s + lane
+    int rank[kDispGroups];          // assignments before this one with its expert
+#pragma unroll
+    for (int g = 0; g < kDispGroups; g++) rank[g] = 0;
+#pragma unroll
+    for (int g = 0; g < kDispGroups; g++) {
+        if (64 * g >= A) break;
+        const uint64_t valid = __ballot(ev[g] >= 0);
+        uint64_t bb[8], mine = valid;  // mine: group g's lanes with expert lane (low 6 bits)
+#pragma unroll
+        for (int b = 0; b < 8; b++) bb[b] = __ballot((ev[g] >> b) & 1);
+#pragma unroll
+        for (int b = 0; b < 6; b++) mine &= ((lane >> b) & 1) ? bb[b] : ~bb[b];
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+            cnt[s] += __popcll(mine & ((s & 1) ? bb[6] : ~bb[6]) & ((s & 2) ? bb[7] : ~bb[7]));
+#pragma unroll
+        for (int h = g; h < kDispGroups; h++) {  // matches of group h's lanes in group g
+            uint64_t m = valid;
+#pragma unroll
+            for (int b = 0; b < 8; b++) m &= ((ev[h] >> b) & 1) ? bb[b] : ~bb[b];
+            rank[h] += __popcll(h == g ? m & below : m);
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+        if (64 * s + lane < E) {
+            a.counts[64 * s + lane] = cnt[s];
+            s_off[64 * s + lane] = cnt[s];
+        }
+    chain_detail::wave_lds_sync();
+    scan_experts(a, s_off);
+    chain_detail::wave_lds_sync();
+#pragma unroll
+    for (int g = 0; g < kDispGroups; g++) {
+        const int q = 64 * g + lane;
+        if (q < A) {
+            const int pos = s_off[ev[g]] + rank[g];
+            a.perm[pos] = q;
+            a.inv[q] = pos;
+        }
+    }
+}
+
 // The same dispatch for one token, by one wave, from its selection sel[0..K)
 // in LDS: its K assignments a = k sorted by expert (the experts are distinct).
 __device__ void dispatch_one(const RouterArgs &a, const int *sel) {
@@ -613,25 +679,26 @@ constexpr int kFastThreads = 512;  // 8 waves: one expert per wave for E = 8
 // row-per-lane kernels and f16 hi/lo pieces + sub-block sums for the
 // matrix-core kernels.  Four threads share a 32-column sub-block, eight
 // columns each, and meet through lane shuffles (NTHR threads, a multiple
-// of 64).  With s_x, the same reads stage the token row into LDS for the
-// logits: lane l's chunk of C = 4*NC4 columns is row l of C + 4 floats,
-// which keeps 8 consecutive lanes' b128 reads on distinct banks.  With
-// nshare > 1 this block takes share `share` of the work (NTHR-thread slices
-// share, share + nshare, ...).
+// of 64).  The row comes from global memory or, with s_x, from LDS as
+// stage_row() lays it out.  With nshare > 1 this block takes share `share`
+// of the work (NTHR-thread slices share, share + nshare, ...).
 template <int NC4, int NTHR = kFastThreads>
-__device__ void quantise_token(const RouterArgs &a, int t, float *s_x, int share = 0,
+__device__ void quantise_token(const RouterArgs &a, int t, const float *s_x, int share = 0,
                                int nshare = 1) {
     constexpr int C = 4 * NC4;
     const int d = a.d, nsb = d / 32;
     for (int q = share * NTHR + threadIdx.x; q < 4 * nsb; q += nshare * NTHR) {
         const int sb = q >> 2, part = q & 3, col0 = 32 * sb + 8 * part;
-        const f32x4 *v = reinterpret_cast<const f32x4 *>(a.x + (int64_t)t * d + col0);
-        const f32x4 v0 = v[0], v1 = v[1];
+        f32x4 v0, v1;
         if (s_x) {
             const int q4 = col0 / 4;
-            *reinterpret_cast<f32x4 *>(s_x + (q4 / NC4) * (C + 4) + 4 * (q4 % NC4)) = v0;
-            *reinterpret_cast<f32x4 *>(s_x + ((q4 + 1) / NC4) * (C + 4) + 4 * ((q4 + 1) % NC4)) =
-                v1;
+            v0 = *reinterpret_cast<const f32x4 *>(s_x + (q4 / NC4) * (C + 4) + 4 * (q4 % NC4));
+            v1 = *reinterpret_cast<const f32x4 *>(s_x + ((q4 + 1) / NC4) * (C + 4) +
+                                                  4 * ((q4 + 1) % NC4));
+        } else {
+            const f32x4 *v = reinterpret_cast<const f32x4 *>(a.x + (int64_t)t * d + col0);
+            v0 = v[0];
+            v1 = v[1];
         }
         const float f[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
         if (a.xh) {
@@ -713,10 +780,10 @@ __device__ __forceinline__ void load_wchunk(const RouterArgs &a, int e, f32x4 (&
 }
 
 template <int NC4>
-__device__ __forceinline__ void logit_bounds(const RouterArgs &a, LogitRegs<NC4> &R, double *s_a,
-                                             double *s_b) {
-    constexpr int W = kFastThreads / 64;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+__device__ __forceinline__ void logit_bounds(const RouterArgs &a, LogitRegs<NC4> &R, int part,
+                                             int nb, double *s_a, double *s_b) {
+    const int W = kFastThreads / 64 * nb;  // waves sharing the token's experts
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) + kFastThreads / 64 * part;
     const int d = a.d, E = a.E, E8 = E & ~7;
     // up to d = 2048 the next expert's chunk loads while this one is summed
     // (a second register set; at larger d it would spill)
@@ -728,6 +795,9 @@ __device__ __forceinline__ void logit_bounds(const RouterArgs &a, LogitRegs<NC4>
             if (more) load_wchunk<NC4>(a, e + W, wn);
         } else {
             if (e != wave) load_wchunk<NC4>(a, e, R.wv);
+            // the row is read again for each expert: kept across them as
+            // float64 (as the compiler does up to d = 2048) it would spill
+            asm volatile("" ::: "memory");
         }
         double l2[2] = {0.0, 0.0}, ab2[2] = {0.0, 0.0}, qg[NC4];
 #pragma unroll
@@ -770,34 +840,92 @@ __device__ __forceinline__ void logit_bounds(const RouterArgs &a, LogitRegs<NC4>
     }
 }
 
-// columns per LDS pass of the fused norm: small, so that its registers fit
-// beside the router chunk already in flight
-constexpr int kFusedNormChunk = 1024;
-
-template <int NC4>
-__device__ __forceinline__ void logits_and_activations(const RouterArgs &a, int t, float *s_x,
-                                                       double *s_a, double *s_b) {
-    LogitRegs<NC4> R;
-    load_wchunk<NC4>(a, min((int)(threadIdx.x >> 6), a.E - 1), R.wv);
-    if (a.xin) {  // the fused norm, while the router chunks load
-        if ((threadIdx.x >> 6) == 0) {
-            const int64_t row = (int64_t)t * a.d;
-            rmsnorm_wave<kFusedNormChunk>(a.xin + row, a.norm_w, a.norm_eps, a.d, a.xn + row, s_x);
+// Token t's row into LDS for the logits: lane l's chunk of C = 4*NC4 columns
+// is row l of C + 4 floats, which keeps 8 consecutive lanes' b128 reads on
+// distinct banks.  With NORM the row of a.xin is first normalised as
+// CpuBackend::rms_norm does, bit for bit (rmsnorm_block's loads, chains and
+// rounding by all the block's threads), and also written to a.xn.  s_x: the
+// chunks, before them the norm's squares (rmsnorm_block_lds(d) floats).
+// Ends without a barrier.
+template <int NC4, bool NORM>
+__device__ __forceinline__ void stage_row(const RouterArgs &a, int t, float *s_x, float *s_scale) {
+    namespace rd = rmsnorm_detail;
+    constexpr int C = 4 * NC4, n4 = 64 * NC4, kPer = (n4 + kFastThreads - 1) / kFastThreads;
+    const int tid = threadIdx.x;
+    const f32x4 *src = reinterpret_cast<const f32x4 *>((NORM ? a.xin : a.x) + (int64_t)t * a.d);
+    f32x4 v[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; k++) v[k] = src[min(tid + kFastThreads * k, n4 - 1)];
+    if constexpr (NORM) {
+        const f32x4 *g = reinterpret_cast<const f32x4 *>(a.norm_w);
+        f32x4 gw[kPer];
+#pragma unroll
+        for (int k = 0; k < kPer; k++) gw[k] = g[min(tid + kFastThreads * k, n4 - 1)];
+        constexpr int ld = n4 + 64 + 4;  // n4 is whole groups of 64: no padding terms
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            const int i = tid + kFastThreads * k;
+            if (i < n4) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) s_x[j * ld + i] = v[k][j] * v[k][j];
+            }
         }
-        __threadfence_block();
         __syncthreads();
+        if (tid < 64) {
+            float acc = 0.0f;
+            if (tid < 4)
+                acc = rd::chain_sum(reinterpret_cast<const float4 *>(s_x + tid * ld), n4 / 4, acc);
+            float sum = 0.0f;
+            for (int j = 0; j < 4; j++) sum = sum + __shfl(acc, j);
+            if (tid == 0) {
+                const float mean = rd::div_rn_pos(sum, (float)a.d);
+                const float root = rd::sqrt_rn(mean + a.norm_eps);
+                *s_scale = root > 0.0f ? rd::div_rn_pos(1.0f, root) : 1.0f / root;
+            }
+        }
+        __syncthreads();
+        const float scale = *s_scale;
+        f32x4 *o = reinterpret_cast<f32x4 *>(a.xn + (int64_t)t * a.d);
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            const int i = tid + kFastThreads * k;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float x = v[k][j] * scale;
+                v[k][j] = x * gw[k][j];
+            }
+            if (i < n4) o[i] = v[k];
+        }
     }
-    quantise_token<NC4>(a, t, s_x);  // while the router chunks load
-    __syncthreads();
-    R.xs = s_x + (threadIdx.x & 63) * (4 * NC4 + 4);
-    logit_bounds<NC4>(a, R, s_a, s_b);
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int i = tid + kFastThreads * k;
+        if (i < n4) *reinterpret_cast<f32x4 *>(s_x + (i / NC4) * (C + 4) + 4 * (i % NC4)) = v[k];
+    }
 }
 
-// grid (T [+ chain blocks]): block t routes token t; with ch.tiles, the
-// blocks past T run the first column range of the exact router chains
-// (wave 0, one tile at a time)
-template <int FBW>
-__global__ __launch_bounds__(kFastThreads) void k_route_fast(RouterArgs a, ChainArgs ch) {
+// part of nb: this block's share of the token's activations and experts
+template <int NC4, bool NORM>
+__device__ __forceinline__ void logits_and_activations(const RouterArgs &a, int t, int part, int nb,
+                                                       float *s_x, float *s_scale, double *s_a,
+                                                       double *s_b) {
+    LogitRegs<NC4> R;
+    load_wchunk<NC4>(a, min((int)(threadIdx.x >> 6) + kFastThreads / 64 * part, a.E - 1), R.wv);
+    stage_row<NC4, NORM>(a, t, s_x, s_scale);  // while the router chunks load
+    __syncthreads();
+    quantise_token<NC4>(a, t, s_x, part, nb);
+    R.xs = s_x + (threadIdx.x & 63) * (4 * NC4 + 4);
+    logit_bounds<NC4>(a, R, part, nb, s_a, s_b);
+}
+
+// grid (T nb [+ chain blocks]): the nb blocks of token t bound every nb-th
+// group of 8 experts each and write a share of the activations; the last of
+// them to finish (a per-token counter, the bounds published through a.bnd)
+// certifies and routes the token, with nb = 1 the block itself.  With
+// ch.tiles, the blocks past T nb run the first column range of the exact
+// router chains (wave 0, one tile at a time).
+template <int FBW, bool NORM>
+__global__ __launch_bounds__(kFastThreads) void k_route_fast(RouterArgs a, ChainArgs ch, int nb) {
     __shared__ double s_a[kMaxE], s_b[kMaxE];
     __shared__ float s_z[kMaxE], s_zlo[kMaxE], s_zhi[kMaxE], s_s[kMaxE], s_g[kMaxE];
     __shared__ int s_sel[kMaxK];
@@ -806,18 +934,20 @@ __global__ __launch_bounds__(kFastThreads) void k_route_fast(RouterArgs a, Chain
     __shared__ int s_flag;
     // x row for the logits (C <= 64 floats per lane), later the fallback's
     // chain stream (one token, 8 experts)
-    // (and first, with the fused norm, its squares: kRmsnormLds floats)
+    // (and first, with the fused norm, its squares)
     // the fallback's chain streams: one region for each of its FBW waves
     constexpr int kXFloats = 64 * (64 + 4), kFbFloats = chain_lds_floats(1 + 8, 256);
     constexpr int kFbAll = kFbFloats * FBW;
     constexpr int kS1 = kXFloats > kFbAll ? kXFloats : kFbAll;
-    constexpr int kS2 = rmsnorm_lds<kFusedNormChunk>();
+    constexpr int kS2 = rmsnorm_block_lds(4096);
     __shared__ __attribute__((aligned(16))) float s_x[kS1 > kS2 ? kS1 : kS2];
+    __shared__ float s_scale;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int t = blockIdx.x, d = a.d, E = a.E, K = a.K;
+    const int t = blockIdx.x / nb, part = blockIdx.x % nb, d = a.d, E = a.E, K = a.K;
     if (t >= a.T) {
+        const int rb = a.T * nb;
         if (wave == 0)
-            for (int tile = t - a.T; tile < ch.tiles; tile += gridDim.x - a.T) {
+            for (int tile = blockIdx.x - rb; tile < ch.tiles; tile += gridDim.x - rb) {
                 if (ch.nt == 1)
                     chain_tile<1, 256, 1>(ch, tile, s_x);
                 else
@@ -832,11 +962,31 @@ __global__ __launch_bounds__(kFastThreads) void k_route_fast(RouterArgs a, Chain
     // 1. activations for the expert products; float64 logit and chain error
     //    bound per expert, one wave each
     switch (d >> 8) {
-    case 1: logits_and_activations<1>(a, t, s_x, s_a, s_b); break;
-    case 2: logits_and_activations<2>(a, t, s_x, s_a, s_b); break;
-    case 4: logits_and_activations<4>(a, t, s_x, s_a, s_b); break;
-    case 8: logits_and_activations<8>(a, t, s_x, s_a, s_b); break;
-    default: logits_and_activations<16>(a, t, s_x, s_a, s_b); break;
+    case 1: logits_and_activations<1, NORM>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
+    case 2: logits_and_activations<2, NORM>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
+    case 4: logits_and_activations<4, NORM>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
+    case 8: logits_and_activations<8, NORM>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
+    default: logits_and_activations<16, NORM>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
+    }
+    if (nb > 1) {  // publish this block's bounds; the token's last block goes on
+        __syncthreads();
+        for (int e = tid; e < E; e += kFastThreads)
+            if (e / (kFastThreads / 64) % nb == part) {
+                uint64_t *out = a.bnd + ((int64_t)t * E + e) * 2;
+                store_agent_u64(out, (uint64_t)__double_as_longlong(s_a[e]));
+                store_agent_u64(out + 1, (uint64_t)__double_as_longlong(s_b[e]));
+            }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tid == 0) s_flag = atomicAdd(&a.tsync[t], 1u) == (unsigned)nb - 1;
+        __syncthreads();
+        if (!s_flag) return;
+        if (tid == 0) a.tsync[t] = 0;
+        for (int e = tid; e < E; e += kFastThreads) {
+            const uint64_t *in = a.bnd + ((int64_t)t * E + e) * 2;
+            s_a[e] = __longlong_as_double((long long)load_agent_u64(in));
+            s_b[e] = __longlong_as_double((long long)load_agent_u64(in + 1));
+        }
     }
     __syncthreads();
 
@@ -934,8 +1084,12 @@ __global__ __launch_bounds__(kFastThreads) void k_route_fast(RouterArgs a, Chain
     }
     __syncthreads();
     if (!s_flag) return;
-    dispatch_block<kFastThreads>(a, s_cw, s_off);
     if (tid == 0) a.sync[0] = 0;
+    if (a.T * a.K <= 64 * kDispGroups) {
+        if (wave == 0) dispatch_wave(a, s_off);
+    } else {
+        dispatch_block<kFastThreads>(a, s_cw, s_off);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -980,14 +1134,6 @@ __host__ __device__ constexpr bool sig_nc4_ok(int n) {
     return n == 1 || n == 2 || n == 4 || n == 8 || n == 16 || n == 28 || n == 32;
 }
 
-__device__ __forceinline__ void store_agent_u64(uint64_t *p, uint64_t v) {
-    __hip_atomic_store(reinterpret_cast<unsigned long long *>(p), (unsigned long long)v,
-                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ uint64_t load_agent_u64(const uint64_t *p) {
-    return __hip_atomic_load(reinterpret_cast<unsigned long long *>(const_cast<uint64_t *>(p)),
-                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // The certification keys of one expert from its chain logit interval
 // [S - B, S + B]: the interval's float ends zlo = up(S - B), zhi = down(S + B)
@@ -1418,8 +1564,12 @@ __global__ __launch_bounds__(64 * kSelWaves) void k_route_select(RouterArgs a) {
     }
     __syncthreads();
     if (!s_flag) return;
-    dispatch_block<64 * kSelWaves>(a, s_cw, s_off);
     if (tid == 0) a.sync[0] = 0;
+    if (a.T * a.K <= 64 * kDispGroups) {
+        if (wave == 0) dispatch_wave(a, s_off);
+    } else {
+        dispatch_block<64 * kSelWaves>(a, s_cw, s_off);
+    }
 }
 
 __global__ void k_debug_sigmoid(const float *__restrict__ x, int64_t n, float *__restrict__ out) {
@@ -1487,6 +1637,21 @@ bool route_fast_ok(const RouterArgs &a) {
            (c4 == 1 || c4 == 2 || c4 == 4 || c4 == 8 || c4 == 16);
 }
 
+// Blocks per token of the fast router: the float64 bounds of E experts are
+// VALU work of the token's CU (60 experts at d = 2048: ~7 us), so while the
+// blocks still fit the CUs side by side, two to eight share a token, each at
+// least 8 experts (its eight waves).  The published bounds and the counter
+// cost ~2 us.  Config 5's router, one block against the split (with the
+// norm's 512-thread form and the one-wave dispatch on both sides of the
+// second figure): T = 16 30 -> 16 us, T = 9 32 -> 16, T = 37 31 -> 20.
+// E <= 8 (one expert per wave) has nothing to share.
+static int fast_split(const RouterArgs &a) {
+    int nb = 1;
+    if (a.T < 2 || !a.bnd || !a.tsync) return nb;
+    while (nb < 8 && a.E > 8 * nb && a.T * nb * 2 <= 256) nb *= 2;
+    return nb;
+}
+
 hipError_t launch_route_fast(const RouterArgs &a, const ChainArgs &ch, hipStream_t st) {
     ChainArgs c = ch;
     int cb = 0;
@@ -1499,10 +1664,11 @@ hipError_t launch_route_fast(const RouterArgs &a, const ChainArgs &ch, hipStream
     // KB; 8 do not fit beside the rest), which leaves one block per CU, so
     // only while the grid fits one round of the CUs; E <= 8 has one tile and
     // keeps the small LDS footprint
-    if (a.E > 8 && a.T <= 256)
-        hipLaunchKernelGGL(k_route_fast<4>, dim3(a.T + cb), dim3(kFastThreads), 0, st, a, c);
-    else
-        hipLaunchKernelGGL(k_route_fast<1>, dim3(a.T + cb), dim3(kFastThreads), 0, st, a, c);
+    const int nb = fast_split(a);
+    const bool wide = a.E > 8 && a.T <= 256;
+    auto *kern = a.xin ? (wide ? k_route_fast<4, true> : k_route_fast<1, true>)
+                       : (wide ? k_route_fast<4, false> : k_route_fast<1, false>);
+    hipLaunchKernelGGL(kern, dim3(a.T * nb + cb), dim3(kFastThreads), 0, st, a, c, nb);
     return hipGetLastError();
 }
 

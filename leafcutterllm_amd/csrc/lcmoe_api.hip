@@ -668,9 +668,9 @@ static lcmoe_status enqueue_forward(lcmoe_handle *h, const float *x, int32_t T, 
     // token the softmax kinds' when E >= kParallelBoundsMinE (the fast
     // router's single block would read the whole router matrix alone).  Its
     // weights, like the fast router's, come from the chains and the combine.
+    ra.bnd = h->sig_bnd;
+    ra.tsync = h->sig_sync;
     RouterArgs rs = ra;
-    rs.bnd = h->sig_bnd;
-    rs.tsync = h->sig_sync;
     rs.flag = h->sig_flag;
     const bool par = T == 1 && E >= kParallelBoundsMinE &&
                      D.route_kind != LCMOE_ROUTE_SIGMOID_GROUP && route_sig_ok(rs);
