@@ -679,26 +679,34 @@ constexpr int kFastThreads = 512;  // 8 waves: one expert per wave for E = 8
 // row-per-lane kernels and f16 hi/lo pieces + sub-block sums for the
 // matrix-core kernels.  Four threads share a 32-column sub-block, eight
 // columns each, and meet through lane shuffles (NTHR threads, a multiple
-// of 64).  The row comes from global memory or, with s_x, from LDS as
-// stage_row() lays it out.  With nshare > 1 this block takes share `share`
+// of 64).  The row comes from global memory (kRowGlobal), from there into
+// LDS too, as stage_row() lays it out (kRowStage), or from LDS (kRowLds).
+// With nshare > 1 this block takes share `share`
 // of the work (NTHR-thread slices share, share + nshare, ...).
-template <int NC4, int NTHR = kFastThreads>
-__device__ void quantise_token(const RouterArgs &a, int t, const float *s_x, int share = 0,
+enum RowFrom { kRowGlobal, kRowStage, kRowLds };
+
+template <int NC4, int NTHR = kFastThreads, RowFrom FROM = kRowGlobal>
+__device__ void quantise_token(const RouterArgs &a, int t, float *s_x, int share = 0,
                                int nshare = 1) {
     constexpr int C = 4 * NC4;
     const int d = a.d, nsb = d / 32;
     for (int q = share * NTHR + threadIdx.x; q < 4 * nsb; q += nshare * NTHR) {
         const int sb = q >> 2, part = q & 3, col0 = 32 * sb + 8 * part;
         f32x4 v0, v1;
-        if (s_x) {
-            const int q4 = col0 / 4;
-            v0 = *reinterpret_cast<const f32x4 *>(s_x + (q4 / NC4) * (C + 4) + 4 * (q4 % NC4));
-            v1 = *reinterpret_cast<const f32x4 *>(s_x + ((q4 + 1) / NC4) * (C + 4) +
-                                                  4 * ((q4 + 1) % NC4));
+        const int q4 = col0 / 4;
+        float *l0 = s_x + (q4 / NC4) * (C + 4) + 4 * (q4 % NC4);
+        float *l1 = s_x + ((q4 + 1) / NC4) * (C + 4) + 4 * ((q4 + 1) % NC4);
+        if constexpr (FROM == kRowLds) {
+            v0 = *reinterpret_cast<const f32x4 *>(l0);
+            v1 = *reinterpret_cast<const f32x4 *>(l1);
         } else {
             const f32x4 *v = reinterpret_cast<const f32x4 *>(a.x + (int64_t)t * d + col0);
             v0 = v[0];
             v1 = v[1];
+        }
+        if constexpr (FROM == kRowStage) {
+            *reinterpret_cast<f32x4 *>(l0) = v0;
+            *reinterpret_cast<f32x4 *>(l1) = v1;
         }
         const float f[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
         if (a.xh) {
@@ -779,10 +787,10 @@ __device__ __forceinline__ void load_wchunk(const RouterArgs &a, int e, f32x4 (&
     for (int i = 0; i < NC4; i++) wv[i] = wr[64 * i];
 }
 
-template <int NC4>
+template <int NC4, bool SHARE>
 __device__ __forceinline__ void logit_bounds(const RouterArgs &a, LogitRegs<NC4> &R, int part,
                                              int nb, double *s_a, double *s_b) {
-    const int W = kFastThreads / 64 * nb;  // waves sharing the token's experts
+    const int W = kFastThreads / 64 * (SHARE ? nb : 1);  // waves sharing the token's experts
     const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) + kFastThreads / 64 * part;
     const int d = a.d, E = a.E, E8 = E & ~7;
     // up to d = 2048 the next expert's chunk loads while this one is summed
@@ -796,8 +804,9 @@ __device__ __forceinline__ void logit_bounds(const RouterArgs &a, LogitRegs<NC4>
         } else {
             if (e != wave) load_wchunk<NC4>(a, e, R.wv);
             // the row is read again for each expert: kept across them as
-            // float64 (as the compiler does up to d = 2048) it would spill
-            asm volatile("" ::: "memory");
+            // float64 it would spill here (the kernel of one block per token
+            // has the registers, and gains 0.7 us at config 2, T = 1)
+            if constexpr (SHARE) asm volatile("" ::: "memory");
         }
         double l2[2] = {0.0, 0.0}, ab2[2] = {0.0, 0.0}, qg[NC4];
 #pragma unroll
@@ -905,20 +914,27 @@ __device__ __forceinline__ void stage_row(const RouterArgs &a, int t, float *s_x
 }
 
 // part of nb: this block's share of the token's activations and experts
-template <int NC4, bool NORM>
+template <int NC4, bool NORM, bool SHARE>
 __device__ __forceinline__ void logits_and_activations(const RouterArgs &a, int t, int part, int nb,
                                                        float *s_x, float *s_scale, double *s_a,
                                                        double *s_b) {
     LogitRegs<NC4> R;
     load_wchunk<NC4>(a, min((int)(threadIdx.x >> 6) + kFastThreads / 64 * part, a.E - 1), R.wv);
-    stage_row<NC4, NORM>(a, t, s_x, s_scale);  // while the router chunks load
-    // a row that is there already: the activations from a second read of it
-    // (cached), not behind the barrier (config 2, T = 1: 58.9 -> 58.1 us)
-    if (!NORM) quantise_token<NC4>(a, t, nullptr, part, nb);
-    __syncthreads();
-    if (NORM) quantise_token<NC4>(a, t, s_x, part, nb);
+    // while the router chunks load: the row into LDS and the activations out
+    if constexpr (NORM) {
+        stage_row<NC4, true>(a, t, s_x, s_scale);
+        __syncthreads();
+        quantise_token<NC4, kFastThreads, kRowLds>(a, t, s_x, part, nb);
+    } else if constexpr (!SHARE) {
+        quantise_token<NC4, kFastThreads, kRowStage>(a, t, s_x);
+        __syncthreads();
+    } else {
+        stage_row<NC4, false>(a, t, s_x, s_scale);
+        quantise_token<NC4>(a, t, nullptr, part, nb);
+        __syncthreads();
+    }
     R.xs = s_x + (threadIdx.x & 63) * (4 * NC4 + 4);
-    logit_bounds<NC4>(a, R, part, nb, s_a, s_b);
+    logit_bounds<NC4, SHARE>(a, R, part, nb, s_a, s_b);
 }
 
 // grid (T nb [+ chain blocks]): the nb blocks of token t bound every nb-th
@@ -926,9 +942,10 @@ __device__ __forceinline__ void logits_and_activations(const RouterArgs &a, int 
 // them to finish (a per-token counter, the bounds published through a.bnd)
 // certifies and routes the token, with nb = 1 the block itself.  With
 // ch.tiles, the blocks past T nb run the first column range of the exact
-// router chains (wave 0, one tile at a time).
-template <int FBW, bool NORM>
+// router chains (wave 0, one tile at a time).  SHARE: nb = 1 << lognb > 1.
+template <int FBW, bool NORM, bool SHARE>
 __global__ __launch_bounds__(kFastThreads) void k_route_fast(RouterArgs a, ChainArgs ch, int lognb) {
+    if (!SHARE) lognb = 0;
     __shared__ double s_a[kMaxE], s_b[kMaxE];
     __shared__ float s_z[kMaxE], s_zlo[kMaxE], s_zhi[kMaxE], s_s[kMaxE], s_g[kMaxE];
     __shared__ int s_sel[kMaxK];
@@ -966,13 +983,13 @@ __global__ __launch_bounds__(kFastThreads) void k_route_fast(RouterArgs a, Chain
     // 1. activations for the expert products; float64 logit and chain error
     //    bound per expert, one wave each
     switch (d >> 8) {
-    case 1: logits_and_activations<1, NORM>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
-    case 2: logits_and_activations<2, NORM>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
-    case 4: logits_and_activations<4, NORM>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
-    case 8: logits_and_activations<8, NORM>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
-    default: logits_and_activations<16, NORM>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
+    case 1: logits_and_activations<1, NORM, SHARE>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
+    case 2: logits_and_activations<2, NORM, SHARE>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
+    case 4: logits_and_activations<4, NORM, SHARE>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
+    case 8: logits_and_activations<8, NORM, SHARE>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
+    default: logits_and_activations<16, NORM, SHARE>(a, t, part, nb, s_x, &s_scale, s_a, s_b); break;
     }
-    if (nb > 1) {  // publish this block's bounds; the token's last block goes on
+    if constexpr (SHARE) {  // publish this block's bounds; the token's last block goes on
         __syncthreads();
         for (int e = tid; e < E; e += kFastThreads)
             if (((e / (kFastThreads / 64)) & (nb - 1)) == part) {
@@ -1499,24 +1516,31 @@ __global__ __launch_bounds__(64 * kSigWaves) void k_route_sig(RouterArgs a, Chai
 // T*E*d makes the per-token fast router re-read the router matrix too often.
 //
 // Launch 1, grid (chain blocks + activation blocks): wave w of chain block b
-// runs tile 4b + w (8 tokens x 8 experts over all d columns); activation
-// block T0 + t prepares token t's limbs and/or f16 pieces.
+// runs tile W b + w (8 tokens x 8 experts over all d columns); activation
+// block T0 + t prepares token t's limbs and/or f16 pieces.  A chain lane
+// reads two float4 from LDS for every four steps, so tile waves that share
+// a CU's LDS slow each other: W = 1 while every tile can have a CU of its
+// own (kChainSpread), else 4.  Both launches together, W = 4 against 1, us:
+// config 4 at T = 32 (128 tiles) 66.9 / 57.1, T = 64 (256) 68.8 / 62.0,
+// T = 150 (608) 73.6 / 74.6, T = 256 (1024) 79.3 / 97.5; config 2 at T = 1000
+// (125) 49.9 / 44.5; config 3 at T = 900 (904) 42.0 / 43.6.
 // Launch 2, grid (ceil(T / 8)): wave w selects token 8b + w from its logits
 // (select_token); the last block to finish dispatches (one token: the
 // selecting wave dispatches from LDS).
 // ---------------------------------------------------------------------------
 
-constexpr int kChainWaves = 4;
 constexpr int kChainLds = chain_lds_floats(9, 256) > chain_lds_floats(16, 128)
                               ? chain_lds_floats(9, 256)
                               : chain_lds_floats(16, 128);
+constexpr int kChainSpread = 256;  // most tiles that get a block each
 constexpr int kSelWaves = 8;
 
-__global__ __launch_bounds__(64 * kChainWaves) void k_route_chains(RouterArgs a, ChainArgs ch,
-                                                                   int chain_blocks) {
-    __shared__ __attribute__((aligned(16))) float s_lds[kChainWaves][kChainLds];
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_route_chains(RouterArgs a, ChainArgs ch,
+                                                         int chain_blocks) {
+    __shared__ __attribute__((aligned(16))) float s_lds[W][kChainLds];
     if ((int)blockIdx.x < chain_blocks) {
-        const int wave = threadIdx.x >> 6, tile = blockIdx.x * kChainWaves + wave;
+        const int wave = threadIdx.x >> 6, tile = blockIdx.x * W + wave;
         // after the certified sigmoid router: only tokens it marked
         bool need = true;
         if (a.flag && tile < ch.tiles) {
@@ -1532,7 +1556,7 @@ __global__ __launch_bounds__(64 * kChainWaves) void k_route_chains(RouterArgs a,
         }
         return;
     }
-    quantise_token<1, 64 * kChainWaves>(a, blockIdx.x - chain_blocks, nullptr);
+    quantise_token<1, 64 * W>(a, blockIdx.x - chain_blocks, nullptr);
 }
 
 __global__ __launch_bounds__(64 * kSelWaves) void k_route_select(RouterArgs a) {
@@ -1622,9 +1646,10 @@ bool route_chains_ok(const RouterArgs &a) { return a.d % 128 == 0 && (a.T >= 8 |
 hipError_t launch_route_chains(const RouterArgs &a, hipStream_t st) {
     const ChainArgs ch =
         make_chains(a.x, a.wrt, a.logits, nullptr, a.T, a.d, a.E, 0, a.d, a.T < 8 ? 1 : 8);
-    const int cb = (ch.tiles + kChainWaves - 1) / kChainWaves;
+    const int W = ch.tiles <= kChainSpread ? 1 : 4, cb = (ch.tiles + W - 1) / W;
     const int ab = (a.xh || a.x16) ? a.T : 0;
-    hipLaunchKernelGGL(k_route_chains, dim3(cb + ab), dim3(64 * kChainWaves), 0, st, a, ch, cb);
+    hipLaunchKernelGGL(W == 1 ? k_route_chains<1> : k_route_chains<4>, dim3(cb + ab), dim3(64 * W),
+                       0, st, a, ch, cb);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_route_select, dim3((a.T + kSelWaves - 1) / kSelWaves),
@@ -1671,8 +1696,9 @@ hipError_t launch_route_fast(const RouterArgs &a, const ChainArgs &ch, hipStream
     // keeps the small LDS footprint
     const int lognb = fast_split(a);
     const bool wide = a.E > 8 && a.T <= 256;
-    auto *kern = a.xin ? (wide ? k_route_fast<4, true> : k_route_fast<1, true>)
-                       : (wide ? k_route_fast<4, false> : k_route_fast<1, false>);
+    auto *kern = lognb  ? (a.xin ? k_route_fast<4, true, true> : k_route_fast<4, false, true>)
+                 : wide ? (a.xin ? k_route_fast<4, true, false> : k_route_fast<4, false, false>)
+                        : (a.xin ? k_route_fast<1, true, false> : k_route_fast<1, false, false>);
     hipLaunchKernelGGL(kern, dim3((a.T << lognb) + cb), dim3(kFastThreads), 0, st, a,
                        c, lognb);
     return hipGetLastError();
