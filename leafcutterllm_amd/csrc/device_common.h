@@ -253,8 +253,8 @@ __device__ __forceinline__ uint32_t ord_key(float f) {
 // column order, as a (hi, lo) pair.  v: the 32 values, 16-byte aligned.
 // Position of column c (0..255) inside its piece of the matrix-core
 // activation format: columns are stored permuted within each group of four
-// as (c0, c2, c1, c3), the order in which one and-or pulls two nibbles out of
-// a packed weight word as f16 magic values (bytes 0 and 2, then 1 and 3).
+// as (c0, c2, c1, c3), the order in which one and pulls two nibbles out of
+// a packed weight word as f16 subnormals (bytes 0 and 2, then 1 and 3).
 // The permutation is applied to both operands of every product, so the sums
 // are unchanged.
 __device__ __forceinline__ int act16_pos(int c) { return (c & ~3) | ((c & 1) << 1) | ((c >> 1) & 1); }

@@ -134,10 +134,11 @@ __device__ __forceinline__ Hdr unpack_hdr_split(u32x4 h, uint32_t db) {
 // q * 2^-24, one and, and one packed multiply by sc * 2^5 makes it
 // sc*q * 2^-19 -- exact: an integer of at most 10 bits times a power of two
 // (subnormal below 32; neither the multiply nor the MFMA flushes those).
-// The high nibbles stay in place as 16 q * 2^-24 and take sc * 2.  (An and-or with the exponent of 1024 and a packed fma that
-// takes 1024 sc away again decode as exactly, the bits of every result the
-// same; both are three-operand instructions, and an and issues at twice an
-// and-or's rate beside another wave's VALU work.  Measured with them before:
+// The high nibbles stay in place as 16 q * 2^-24 and take sc * 2.  (An and-or
+// with the exponent of 1024 and a packed fma that takes 1024 sc away again
+// decode as exactly, the bits of every result the same; both are
+// three-operand instructions, and an and issues at twice an and-or's rate
+// beside another wave's VALU work.  Measured with them before:
 // config 3 T = 1801 gate/up 262 -> 249 us, down 156 -> 150; config 2
 // T = 1000 621 -> 605; config 5's layer at T = 16, two f16 per activation,
 // 96.3 -> 94.1 us per call; config 2 T = 64 within 1%.)
