@@ -8,7 +8,8 @@
 // Each chain is
 // sequential, so a chain occupies one lane; a wave runs the NT x 8
 // (token, expert) chains of one tile, lane l taking token t0 + l / 8 (NT = 8)
-// or t0 (NT = 1) and expert e0 + l % 8.  Indices past T or E are clamped to
+// or t0 (NT = 1) and expert e0 + l % 8 (NT = 1 also with NE = 32 experts,
+// lane l taking e0 + l % 32).  Indices past T or E are clamped to
 // the last valid one for the loads and their results are dropped.
 //
 // The NT x rows and 8 router rows advance together in chunks of CH columns:
@@ -121,16 +122,17 @@ __device__ __forceinline__ void wave_lds_sync() {
 }  // namespace chain_detail
 
 // One wave's tile `tile` of chains over columns [a.k0, a.k1); lds:
-// chain_lds_floats(NT + 8, CH) floats private to this wave.  Requires k0 and
+// chain_lds_floats(NT + NE, CH) floats private to this wave.  Requires k0 and
 // k1 to be multiples of CH.
-template <int NT, int CH, int DEPTH>
+template <int NT, int CH, int DEPTH, int NE = 8>
 __device__ void chain_tile(const ChainArgs &a, int tile, float *lds) {
     using namespace chain_detail;
-    constexpr int NR = NT + 8, ROW = CH + 4, F4 = CH / 4;  // float4 per row per chunk
-    constexpr int NL = NR * F4 / 64;                       // loads per lane per chunk
-    static_assert(NR * F4 % 64 == 0, "chunk must split evenly over the wave");
-    const int lane = threadIdx.x & 63, ne = (a.E + 7) / 8;
-    const int t0 = (tile / ne) * NT, e0 = (tile % ne) * 8;
+    constexpr int NR = NT + NE, ROW = CH + 4, F4 = CH / 4;  // float4 per row per chunk
+    // loads per lane per chunk; the last may repeat the chunk's last float4
+    constexpr int NL = (NR * F4 + 63) / 64;
+    static_assert(NE == 8 || NT == 1, "a lane per chain");
+    const int lane = threadIdx.x & 63, ne = (a.E + NE - 1) / NE;
+    const int t0 = (tile / ne) * NT, e0 = (tile % ne) * NE;
     const int nch = (a.k1 - a.k0) / CH;
     // the chain is one long dependency: issue its instructions ahead of the
     // streaming waves that share this SIMD
@@ -140,7 +142,7 @@ __device__ void chain_tile(const ChainArgs &a, int tile, float *lds) {
     int dst[NL];
 #pragma unroll
     for (int i = 0; i < NL; i++) {
-        const int j = i * 64 + lane, r = j / F4, c4 = j % F4;
+        const int j = min(i * 64 + lane, NR * F4 - 1), r = j / F4, c4 = j % F4;
         const float *row = r < NT ? a.x + (int64_t)min(t0 + r, a.T - 1) * a.d
                                   : a.wrt + (int64_t)min(e0 + r - NT, a.E - 1) * a.d;
         src[i] = reinterpret_cast<const f32x4 *>(row + a.k0) + c4;
@@ -157,7 +159,7 @@ __device__ void chain_tile(const ChainArgs &a, int tile, float *lds) {
     for (int i = 0; i < NL; i++) v[0][i] = src[i][min(DEPTH, nch - 1) * F4];
     wave_lds_sync();
 
-    const int tb = NT == 1 ? 0 : lane / 8, eg = lane % 8;
+    const int tb = NT == 1 ? 0 : lane / 8, eg = lane % NE;
     const bool fma = min(e0 + eg, a.E - 1) < (a.E & ~7);
     const int xoff = tb * ROW, woff = (NT + eg) * ROW;
     const int t = t0 + tb, e = e0 + eg;
@@ -189,7 +191,7 @@ __device__ void chain_tile(const ChainArgs &a, int tile, float *lds) {
         }
     }
     float *out = a.k1 < a.d ? a.part : a.logits;
-    if (t < a.T && e < a.E && (NT == 8 || lane < 8)) out[(int64_t)t * a.E + e] = acc;
+    if (t < a.T && e < a.E && (NT == 8 || lane < NE)) out[(int64_t)t * a.E + e] = acc;
     __builtin_amdgcn_s_setprio(0);
 }
 

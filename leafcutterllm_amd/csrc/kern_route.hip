@@ -1454,9 +1454,18 @@ template <int NC4, int FBW>
 __global__ __launch_bounds__(64 * kSigWaves) void k_route_sig(RouterArgs a, ChainArgs ch) {
     __shared__ float s_f[3 * kMaxE + 3 * 64];  // certification: keys, group scores
     // one wave's chain stream: the chain blocks', or the one-token fallback's
-    // streams, one for each of its FBW waves
+    // streams, one for each of its FBW waves.  Those are tiles of 32 experts:
+    // every lane of a wave reads its LDS rows whether it owns a chain or not,
+    // so a tile of 32 takes little longer than one of 8, and the block's four
+    // waves go over 256 experts twice instead of eight times (config 4's layer
+    // at one uncertified token 362 -> 200 us; certified tokens 79 -> 80).
+    // The LDS (139 KB) leaves one block per CU; one token needs at most 128.
+    constexpr int kFbCols = 128, kFbExperts = 32;
     constexpr int kChainFloats = chain_lds_floats(1 + 8, 256);
-    __shared__ __attribute__((aligned(16))) float s_chain[kChainFloats * FBW];
+    constexpr int kFbFloats = chain_lds_floats(1 + kFbExperts, kFbCols);
+    constexpr int kFbAll = FBW > 1 ? kFbFloats * FBW : 0;
+    __shared__ __attribute__((aligned(16))) float
+        s_chain[kFbAll > kChainFloats ? kFbAll : kChainFloats];
     __shared__ int s_last;
     const int t = blockIdx.y, tid = threadIdx.x, wave = tid >> 6;
     const int nsig = a.E / kSigWaves;  // bound blocks per token
@@ -1488,15 +1497,15 @@ __global__ __launch_bounds__(64 * kSigWaves) void k_route_sig(RouterArgs a, Chai
     if (a.T > 1) return;  // the chains, selection and dispatch launches follow
     // one token: this block finishes the routing itself (no launches
     // follow): for an uncertified token the exact chains over all d columns
-    // (its tiles of 8 experts spread over FBW waves) and the exact
+    // (its tiles of 32 experts spread over FBW waves) and the exact
     // selection, then the dispatch from LDS
     __syncthreads();
     if (!s_ok) {
-        if (wave < FBW) {
+        if constexpr (FBW > 1) {
             const ChainArgs ca = make_chains(a.x, a.wrt, a.logits, nullptr, a.T, a.d, a.E, 0,
                                              a.d, 1);
-            for (int g = wave; g < ca.tiles; g += FBW)
-                chain_tile<1, 256, 1>(ca, g, s_chain + wave * kChainFloats);
+            for (int g = wave; g < (a.E + kFbExperts - 1) / kFbExperts; g += FBW)
+                chain_tile<1, kFbCols, 2, kFbExperts>(ca, g, s_chain + wave * kFbFloats);
         }
         __threadfence_block();
         __syncthreads();
