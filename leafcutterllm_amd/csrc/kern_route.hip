@@ -951,7 +951,10 @@ __global__ __launch_bounds__(kFastThreads) void k_route_fast(RouterArgs a, Chain
     __shared__ int s_sel[kMaxK];
     __shared__ int s_cw[kFastThreads / 64][kMaxE];
     __shared__ int s_off[kMaxE + 1];
-    __shared__ int s_flag;
+    // s_flag: the verdict; s_last: the counters' outcome.  The verdict keeps a
+    // variable of its own: a wave may still have to read it when wave 0 is
+    // past the next counter.
+    __shared__ int s_flag, s_last;
     // x row for the logits (C <= 64 floats per lane), later the fallback's
     // chain stream (one token, 8 experts)
     // (and first, with the fused norm, its squares)
@@ -999,9 +1002,9 @@ __global__ __launch_bounds__(kFastThreads) void k_route_fast(RouterArgs a, Chain
             }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        if (tid == 0) s_flag = atomicAdd(&a.tsync[t], 1u) == (unsigned)nb - 1;
+        if (tid == 0) s_last = atomicAdd(&a.tsync[t], 1u) == (unsigned)nb - 1;
         __syncthreads();
-        if (!s_flag) return;
+        if (!s_last) return;
         if (tid == 0) a.tsync[t] = 0;
         for (int e = tid; e < E; e += kFastThreads) {
             const uint64_t *in = a.bnd + ((int64_t)t * E + e) * 2;
@@ -1101,10 +1104,10 @@ __global__ __launch_bounds__(kFastThreads) void k_route_fast(RouterArgs a, Chain
     // published with coherent stores and have completed)
     if (tid == 0) {
         const unsigned old = atomicAdd(&a.sync[0], 1u);
-        s_flag = (old == (unsigned)a.T - 1);
+        s_last = (old == (unsigned)a.T - 1);
     }
     __syncthreads();
-    if (!s_flag) return;
+    if (!s_last) return;
     if (tid == 0) a.sync[0] = 0;
     if (a.T * a.K <= 64 * kDispGroups) {
         if (wave == 0) dispatch_wave(a, s_off);

@@ -27,6 +27,26 @@ def test_split_router_parity(d, E, K, T):
     run_and_check(cfg, layer, L.synth_x(cfg, T, seed=T, index=d))
 
 
+# certified tokens and tokens that fall back side by side in one launch: experts
+# 1 and 2 share a row, which leads for every odd token (no bound orders the
+# pair) and comes last for the others.  One block per token and several.
+@pytest.mark.parametrize("T", [2, 17, 100, 130, 257])
+@pytest.mark.parametrize("d,E,K", [(256, 8, 2), (512, 16, 4), (1024, 60, 4), (2048, 64, 2)])
+def test_certified_and_exact_tokens_together(d, E, K, T):
+    cfg = _cfg(d, E, K)
+    layer = L.synth_layer(cfg, seed=d + T)
+    x = L.synth_x(cfg, T, seed=T, index=d)
+    u = np.where(np.arange(d) % 2, 1.0, -1.0).astype(np.float32) / np.float32(np.sqrt(d))
+    router = layer["router"].copy()
+    router[:, 1] = router[:, 2] = u
+    layer["router"] = router
+    x -= np.outer(x @ u, u)
+    x += np.outer(np.where(np.arange(T) % 2, 8.0, -8.0), u)
+    idx = run_and_check(cfg, layer, x.astype(np.float32))["topk_idx"].reshape(T, K)
+    assert np.all(idx[1::2, :2] == [1, 2])
+    assert not np.any(np.isin(idx[::2], [1, 2]))
+
+
 @pytest.mark.parametrize("d", [256, 512, 1024, 2048, 4096])
 @pytest.mark.parametrize("E,T", [(8, 5), (40, 5), (40, 70)])
 def test_fused_norm_router_is_the_separate_norm(d, E, T):
