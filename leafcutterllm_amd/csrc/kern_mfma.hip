@@ -10,7 +10,7 @@
 // so every per-row quantity (super-block scales d / dmin, 6-bit sub-block
 // scales and mins) is lane-local.
 //
-// Exact operands: B = sc_j * q * 2^-19 (6-bit * 4-bit integers, exact in
+// Exact operands: B = sc_j * q * 2^-14 (6-bit * 4-bit integers, exact in
 // f16), built from the nibbles as f16 subnormals and one packed-f16 multiply
 // (dec_pair).  Activations enter as one f16 per
 // element (LO = false, the default mode) or as two f16 halves hi + lo
@@ -98,7 +98,7 @@ constexpr uint32_t kSel11 = 0x04010401u;
 constexpr uint32_t kSel22 = 0x04020402u;
 constexpr uint32_t kSel33 = 0x04030403u;
 
-constexpr float kDecUnit = 524288.0f;  // dec_pair's operands are sc*q / kDecUnit
+constexpr float kDecUnit = 16384.0f;  // dec_pair's operands are sc*q / kDecUnit
 
 // Per-row super-block header (d, dmin, 12 packed scale bytes) unpacked, d
 // times kDecUnit; d2, dmin2: the scales of sub-blocks 4-7 in the split layout.
@@ -129,30 +129,31 @@ __device__ __forceinline__ Hdr unpack_hdr_split(u32x4 h, uint32_t db) {
     return s;
 }
 
-// Weight operands are sc*q scaled by 2^-19 (Hdr::d carries 2^19 back): a
+// Weight operands are sc*q scaled by 2^-14 (Hdr::d carries 2^14 back): a
 // nibble left in the low bits of a 16-bit half is the f16 subnormal
-// q * 2^-24, one and, and one packed multiply by sc * 2^5 makes it
-// sc*q * 2^-19 -- exact: an integer of at most 10 bits times a power of two
-// (subnormal below 32; neither the multiply nor the MFMA flushes those).
-// The high nibbles stay in place as 16 q * 2^-24 and take sc * 2.  (An and-or
-// with the exponent of 1024 and a packed fma that takes 1024 sc away again
-// decode as exactly, the bits of every result the same; both are
-// three-operand instructions, and an and issues at twice an and-or's rate
-// beside another wave's VALU work.  Measured with them before:
+// q * 2^-24, one and, and one packed multiply by sc * 2^10 makes it the
+// normal number sc*q * 2^-14 -- exact: an integer of at most 10 bits times a
+// power of two.  The high nibbles stay in place as 16 q * 2^-24 and take
+// sc * 2^6.  (An and-or with the exponent of 1024 and a packed fma that
+// takes 1024 sc away again decode as exactly, the bits of every result the
+// same; both are three-operand instructions, and an and issues at twice an
+// and-or's rate beside another wave's VALU work.  Measured with them before:
 // config 3 T = 1801 gate/up 262 -> 249 us, down 156 -> 150; config 2
 // T = 1000 621 -> 605; config 5's layer at T = 16, two f16 per activation,
-// 96.3 -> 94.1 us per call; config 2 T = 64 within 1%.)
+// 96.3 -> 94.1 us per call; config 2 T = 64 within 1%.)  The unit keeps every
+// operand normal: at 2^-19, where a pair's scales take one instruction less,
+// products below 2^-14 are f16 subnormals, and the matrix instruction then
+// rounds some sums otherwise (the decoder's logits no longer the same bits).
 
-// Scales of pair p: (sc_2p * 2^5, sc_2p+1 * 2): a byte under the exponent of
-// 2^15 (0x78) counts 2^5, under that of 2^11 (0x68) two
+// Scales of pair p: (sc_2p * 2^10, sc_2p+1 * 2^6), exact in f16
 __device__ __forceinline__ half2v pair_scales(const Hdr &s, int p) {
     const uint32_t w = p < 2 ? s.sc03 : s.sc47;
-    const uint32_t sel = (p & 1) ? 0x05030402u : 0x05010400u;
-    return as_h2(__builtin_amdgcn_perm(0x00006878u, w, sel)) -
-           half2v{(_Float16)32768.0f, (_Float16)2048.0f};
+    const half2v mag = magic2(w, (p & 1) ? kSel23 : kSel01);  // 1024 + sc
+    return (mag - half2v{(_Float16)1024.0f, (_Float16)1024.0f}) *
+           half2v{(_Float16)1024.0f, (_Float16)64.0f};
 }
 
-// B operands (sc*q * 2^-19, 8 columns each) of pair p's two sub-blocks from
+// B operands (sc*q * 2^-14, 8 columns each) of pair p's two sub-blocks from
 // one lane's 8 qs bytes w0, w1 (bytes j = columns j), in the activation
 // format's column order (act16_pos): bytes 0, 2, 1, 3, 4, 6, 5, 7.  The
 // shifted words w >> 8 bring bytes 1 and 3 down to the places of 0 and 2.
@@ -740,23 +741,14 @@ __device__ __forceinline__ void read_a16(AUnit &a, const uint8_t *tokrow, int p,
 // One step of a 16-token pass (same pipeline as step()).  Per pair p the
 // activations of sub-blocks 2p and 2p+1 (hi, lo) are read once and shared by
 // both tiles and all matrices.
-// PACK (two f16 per activation, at most 8 tokens): rows 0-7 of the A operand
-// are the tokens' hi halves and rows 8-15 their lo halves, so one MFMA takes
-// both where a 16-token pass issues two; the result rows q and q + 8 add up
-// to token q's (fold_packed), and the min term rides with rows 0-7 alone.
-// Config 5's layer, two f16 per activation, gate/up: T = 9 35.6 -> 33.7 us,
-// T = 16 42.5 -> 41.5.
-template <int MATS, bool SPLIT = false, bool LO = true, bool PACK = false>
+template <int MATS, bool SPLIT = false, bool LO = true>
 __device__ __forceinline__ void step16(g_u8 *const (&wb)[MATS], uint32_t lo,
                                        const uint32_t (&dbo)[MATS], int kn, const uint8_t *cur,
                                        uint8_t *nxt, const StageSrc &src, WRaw16 (&w)[MATS],
                                        float4v (&acc)[MATS][2], int wave, int lane) {
-    static_assert(!PACK || LO, "only hi and lo halves pack");
-    constexpr int NI = PACK ? 2 : 4;          // tokens this wave stages
-    constexpr bool LOM = LO && !PACK;         // lo halves take MFMAs of their own
     const int r16 = lane & 15, c4 = lane >> 4;
-    StageRegs<NI, LO> act;
-    stage_load<NI, LO>(act, src, kn, wave, lane);
+    StageRegs<4, LO> act;
+    stage_load<4, LO>(act, src, kn, wave, lane);
     __builtin_amdgcn_sched_barrier(0);  // keep the activation loads first
     Hdr hd[MATS][2];
 #pragma unroll
@@ -770,15 +762,13 @@ __device__ __forceinline__ void step16(g_u8 *const (&wb)[MATS], uint32_t lo,
     float4v S[MATS][2];
 #pragma unroll
     for (int m = 0; m < MATS; m++) S[m][0] = S[m][1] = float4v{};
-    const uint8_t *tokrow = PACK ? cur + (r16 & 7) * kTokB<LO> + (r16 >> 3) * 512
-                                 : cur + r16 * kTokB<LO>;
+    const uint8_t *tokrow = cur + r16 * kTokB<LO>;
     const half4 *aminp = reinterpret_cast<const half4 *>(cur + kSumsOffT<LO> + r16 * 32 + 8 * c4);
-    const auto read_min = [&] { return PACK && r16 >= 8 ? half4{} : *aminp; };
     AUnit a[2];  // pair p's operands, and pair p+1's read ahead
-    read_a16<LOM>(a[0], tokrow, 0, c4);
+    read_a16<LO>(a[0], tokrow, 0, c4);
 #pragma unroll
     for (int p = 0; p < 4; p++) {
-        if (p + 1 < 4) read_a16<LOM>(a[(p + 1) & 1], tokrow, p + 1, c4);
+        if (p + 1 < 4) read_a16<LO>(a[(p + 1) & 1], tokrow, p + 1, c4);
         const half8 h0 = a[p & 1].h0, l0 = a[p & 1].l0, h1 = a[p & 1].h1, l1 = a[p & 1].l1;
 #pragma unroll
         for (int m = 0; m < MATS; m++)
@@ -788,12 +778,12 @@ __device__ __forceinline__ void step16(g_u8 *const (&wb)[MATS], uint32_t lo,
                 dec_pair(hd[m][t], p, w[m].q[p][t].x, w[m].q[p][t].y, blo, bhi);
                 w[m].q[p][t] = load_q16<SPLIT>(wb[m], lo, kn, p, t, c4);
                 S[m][t] = mfma16(h0, blo, S[m][t]);
-                if constexpr (LOM) S[m][t] = mfma16(l0, blo, S[m][t]);
+                if constexpr (LO) S[m][t] = mfma16(l0, blo, S[m][t]);
                 S[m][t] = mfma16(h1, bhi, S[m][t]);
-                if constexpr (LOM) S[m][t] = mfma16(l1, bhi, S[m][t]);
+                if constexpr (LO) S[m][t] = mfma16(l1, bhi, S[m][t]);
             }
         if (SPLIT && p == 1) {  // sub-blocks 0-3 done: their own d, dmin
-            const half4 amin = read_min();
+            const half4 amin = *aminp;
 #pragma unroll
             for (int m = 0; m < MATS; m++)
 #pragma unroll
@@ -804,7 +794,7 @@ __device__ __forceinline__ void step16(g_u8 *const (&wb)[MATS], uint32_t lo,
         }
         __builtin_amdgcn_sched_barrier(0);  // bounds the live operands to two pairs
     }
-    const half4 amin = read_min();
+    const half4 amin = *aminp;
 #pragma unroll
     for (int m = 0; m < MATS; m++)
 #pragma unroll
@@ -814,24 +804,13 @@ __device__ __forceinline__ void step16(g_u8 *const (&wb)[MATS], uint32_t lo,
             else
                 finish16(hd[m][t], amin, c4, S[m][t], acc[m][t]);
         }
-    stage_store<NI, LO>(nxt, act, wave, lane);
+    stage_store<4, LO>(nxt, act, wave, lane);
     lds_barrier();
-}
-
-// token q's sums from the packed rows q and q + 8 (lanes c4 and c4 ^ 2)
-template <int MATS>
-__device__ __forceinline__ void fold_packed(float4v (&acc)[MATS][2]) {
-#pragma unroll
-    for (int m = 0; m < MATS; m++)
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) acc[m][t][i] += __shfl_xor(acc[m][t][i], 32, 64);
 }
 
 // block_pass() for a pass of at most 16 tokens; lo is the offset of this
 // lane's row r16 of the wave's first tile
-template <int MATS, bool SPLIT = false, bool LO = true, bool PACK = false>
+template <int MATS, bool SPLIT = false, bool LO = true>
 __device__ __forceinline__ void block_pass16(g_u8 *const (&wb)[MATS], uint32_t lo,
                                              const uint32_t (&dbo)[MATS], int kb0, int kb1,
                                              const StageSrc &src, float4v (&acc)[MATS][2]) {
@@ -840,22 +819,20 @@ __device__ __forceinline__ void block_pass16(g_u8 *const (&wb)[MATS], uint32_t l
     const int last = kb1 - 1;
     asm volatile("" : "+s"(kb0));  // see block_pass()
     WRaw16 w[MATS];
-    constexpr int NI = PACK ? 2 : 4;
-    StageRegs<NI, LO> act;
-    stage_load<NI, LO>(act, src, kb0, wave, lane);
+    StageRegs<4, LO> act;
+    stage_load<4, LO>(act, src, kb0, wave, lane);
 #pragma unroll
     for (int m = 0; m < MATS; m++) load_w16<SPLIT>(w[m], wb[m], lo, dbo[m], kb0, c4);
-    stage_store<NI, LO>(s_stage0, act, wave, lane);
+    stage_store<4, LO>(s_stage0, act, wave, lane);
     lds_barrier();
     int kb = kb0;
     for (; kb + 2 <= kb1; kb += 2) {
-        step16<MATS, SPLIT, LO, PACK>(wb, lo, dbo, kb + 1, s_stage0, s_stage1, src, w, acc, wave, lane);
-        step16<MATS, SPLIT, LO, PACK>(wb, lo, dbo, min(kb + 2, last), s_stage1, s_stage0, src, w, acc,
+        step16<MATS, SPLIT, LO>(wb, lo, dbo, kb + 1, s_stage0, s_stage1, src, w, acc, wave, lane);
+        step16<MATS, SPLIT, LO>(wb, lo, dbo, min(kb + 2, last), s_stage1, s_stage0, src, w, acc,
                                 wave, lane);
     }
     if (kb < kb1)
-        step16<MATS, SPLIT, LO, PACK>(wb, lo, dbo, kb, s_stage0, s_stage1, src, w, acc, wave, lane);
-    if constexpr (PACK) fold_packed<MATS>(acc);
+        step16<MATS, SPLIT, LO>(wb, lo, dbo, kb, s_stage0, s_stage1, src, w, acc, wave, lane);
 }
 
 // split v into f16 hi + lo
@@ -987,10 +964,7 @@ __global__ __launch_bounds__(256, 2) void k_mfma_gateup(
         if (n - c <= 16) {
             const int r16 = lane & 15, c4 = lane >> 4;
             float4v acc[2][2] = {};
-            if (LO && n - c <= 8)
-                block_pass16<2, false, LO, LO>(wb, r16 * 16, nodb, 0, NB, src, acc);
-            else
-                block_pass16<2, false, LO>(wb, r16 * 16, nodb, 0, NB, src, acc);
+            block_pass16<2, false, LO>(wb, r16 * 16, nodb, 0, NB, src, acc);
             if (grp0 >= ngrp) continue;
             // output addresses are formed here from an opaque row index, so
             // that the compiler does not keep them live across the pass
@@ -1160,11 +1134,7 @@ __global__ __launch_bounds__(256, 2) void k_mfma_down(
             const uint32_t dbo[2] = {9 * 1024 + 4 * (uint32_t)r16,
                                      9 * 1024 + 4 * (32 + (uint32_t)r16) - 32 * 16};
             float4v acc[2][2] = {};
-            // (the split layout's kernel has no registers left for this form)
-            if (LO && !SPLIT && n - c <= 8)
-                block_pass16<2, SPLIT, LO, LO && !SPLIT>(wb, r16 * 16, dbo, kb0, kb1, src, acc);
-            else
-                block_pass16<2, SPLIT, LO>(wb, r16 * 16, dbo, kb0, kb1, src, acc);
+            block_pass16<2, SPLIT, LO>(wb, r16 * 16, dbo, kb0, kb1, src, acc);
             if (tile0 >= ntile) continue;
             int rb = tile * 64 + r16;  // opaque: output addresses are formed here
             asm volatile("" : "+v"(rb));

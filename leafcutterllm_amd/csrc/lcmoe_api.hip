@@ -254,15 +254,12 @@ int choose_ksplit(const ExpertSet &s, int d, int active) {
 }
 
 // Matrix-core down: 256-row blocks, two resident per CU; split K until
-// about four blocks per CU exist, keeping >= 3 super-blocks per split (config
-// 5's F = 1408 is six: down at T = 9 27.8 -> 23.1 us, at T = 16 28.2 -> 26.8,
-// with the combine's extra partials 92 -> 88 and 99.5 -> 98.9 us per layer;
-// config 2 is at its four splits either way, config 4's F = 2048 at two).
+// about two blocks per CU exist, keeping >= 4 super-blocks per split.
 int choose_ksplit_mfma(const ExpertSet &s, int d, int active) {
     if (!s.rpl_dn && !s.q6_dn && !s.split_dn) return 1;
     const int NB = (s.F + 255) / 256, blocks = ((d / 64 + 3) / 4) * std::max(1, active);
     int ks = 1;
-    while (ks < s.kmax && blocks * ks < 1024 && NB >= 3 * ks * 2) ks *= 2;
+    while (ks < s.kmax && blocks * ks < 512 && NB >= 4 * ks * 2) ks *= 2;
     return ks;
 }
 

@@ -6,6 +6,8 @@ Bar: last-token logits within 1e-3 relative L2 of the oracle at every
 forward (prefill and decode, teacher-forced on the same ids); greedy ids
 identical to the oracle's except from a step whose top-2 logits are within
 rounding of each other (none occur in these cases; the check says so)."""
+import functools
+
 import numpy as np
 import pytest
 
@@ -18,6 +20,11 @@ from test_oracle_engine import TINY, rel, spec
 pytestmark = pytest.mark.gpu
 
 LOGIT_TOL = 1e-3
+
+
+@functools.lru_cache(maxsize=1)
+def _config5_cut(n_layer):
+    return synth_model(MODEL_CONFIGS[5], seed=11, n_layer=n_layer)
 
 
 def assert_same_greedy(got, ref, trace):
@@ -147,6 +154,56 @@ def test_config5_two_layer_cut():
                 e = rel(lg[b], refs[b][1][i].astype(np.float64))
                 print(f"config-5 cut step {i} seq {b}: logits rel-L2 {e:.2e}", flush=True)
                 assert e < LOGIT_TOL
+
+
+@pytest.mark.parametrize("B,P", [(2, 2), (3, 5), (2, 13), (8, 4)])
+def test_config5_short_prompts_decoded_together(B, P):
+    """A few short prompts of the config-5 model cut to four layers, then
+    decode steps of B rows on given ids, every row against the oracle up to
+    the first token that a layer routes to different experts there.  Both
+    sides route by logits that carry their own rounding (the f16 cache and,
+    below 4 rows, 15-bit activations: 1.5e-4 of the logits), and a top-k
+    selection is discontinuous, so such a token must be a near-tie; nothing
+    after it is comparable."""
+    from test_gpu_config5_full import assert_near_tie, first_swap
+    mc, NL, N = MODEL_CONFIGS[5], 4, 4
+    w = _config5_cut(NL)
+    tok = np.random.default_rng(100 * B + P).integers(0, mc.vocab, (B, P + N))
+
+    def routing(m):
+        return [m.layer_routing(l) for l in range(NL)]
+
+    with L.Model(mc.desc(8, 16, 32, E.ROPE_ABSOLUTE, n_layer=NL), w) as m:
+        alone, r0 = [], []
+        for b in range(B):  # a prompt alone takes the same launches
+            m.reset()
+            alone.append(m.forward(tok[b:b + 1, :P])[0])
+            r0.append(routing(m))
+        m.reset()
+        lg, rt = [m.forward(tok[:, :P])], [None]
+        assert np.array_equal(lg[0], np.stack(alone))
+        for i in range(P, P + N):
+            lg.append(m.forward(tok[:, i:i + 1]))
+            rt.append(routing(m))
+    ref, compared = E.RefEngine(spec(mc, E.ROPE_ABSOLUTE, n_layer=NL), w, threads=16), 0
+    ref.record_routing = True
+    for b in range(B):
+        ref.clear()
+        for i in range(N + 1):
+            ref.routing = []
+            r = ref.forward([int(t) for t in (tok[b, :P] if i == 0 else tok[b, P + i - 1:P + i])])
+            swaps = [first_swap(r0[b] if i == 0 else rt[i], ref.routing,
+                                row_a=q if i == 0 else b, row_b=q) for q in range(P if i == 0 else 1)]
+            swaps = sorted(x for x in swaps if x is not None)
+            if swaps:  # the first layer's are near-ties; deeper ones may follow from them
+                for x in swaps:
+                    if x[0] == swaps[0][0]:
+                        assert_near_tie(x, (b, i))
+                break
+            e = rel(lg[i][b], r.astype(np.float64))
+            assert e < LOGIT_TOL, (b, i, e)
+            compared += 1
+    assert compared >= B * (N + 1) // 2
 
 
 def test_eager_decode_equals_graph():
