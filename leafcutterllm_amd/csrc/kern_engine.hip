@@ -10,7 +10,7 @@
 //                  f16 KV cache append (cache/mod.rs:33-63)
 //   k_attn_part /  masked softmax attention (attention.rs:56-115), split
 //   k_attn_combine over 128-position chunks of the context, then merged
-//   k_attn_prefill the same for a prompt's tokens on the matrix cores
+//   k_attn_tile    k_attn_part for four tokens of a prompt at a time
 //   k_argmax       greedy sample_top_p (sampler.rs:8-10): max_by(total_cmp),
 //                  the last of equal maxima
 //   k_advance      the cache length after a forward
@@ -27,11 +27,14 @@ namespace lcmoe {
 namespace {
 
 constexpr int kAttnChunk = 128;  // context positions per attention partial
-// Fewest tokens of one sequence that take k_attn_prefill (below, its 32-query
-// tiles are mostly padding; two prompts and two decode steps of the config-5
-// shapes, us, partials + combine against it: 16 tokens 1414 / 1356, 32 tokens
-// 1459 / 1519 before and after on boxes 4% apart).
-constexpr int kPrefillMin = 16;
+// Fewest tokens of one sequence that take k_attn_tile: from here on it is the
+// faster one at every head size and context measured.  k_attn_part against it,
+// with the combine, us: 16 heads x 128 on an empty cache of 512, 16 / 32 / 37 /
+// 48 tokens 8.5 / 10.2, 9.9 / 11.0, 11.7 / 11.3, 11.5 / 11.5; of 8192, 16 / 24
+// / 32 tokens 26 / 31, 36 / 35, 38 / 34; 32 heads x 64, 24 tokens 10.4 / 10.1;
+// 8 heads x 32, 32 / 100 tokens 8.4 / 9.1, 11.9 / 10.2.  (On 2000 cached tokens
+// it would pay from 8 tokens on; the length is device data here.)
+constexpr int kTileMin = 40;
 
 template <int QT>
 __device__ __forceinline__ void dec8(const uint8_t *row, int64_t k, float (&w)[8]) {
@@ -389,246 +392,129 @@ __global__ __launch_bounds__(256) void k_attn_combine(const float *__restrict__ 
     if (sb < hd / 32) act16_subblock(s_o + 32 * sb, q, H * hd, h * (hd / 32) + sb, x16, xs);
 }
 
-// Prompt attention: a block takes 32 queries of one head (tokens i0 .. i0+31
-// of one sequence) and its eight waves every eighth 32-key tile of the
-// context, each with its own running maximum and sums, merged at the end
-// (the log-sum-exp of k_attn_combine); one launch, no partials in memory.
-// Both products run on v_mfma_f32_32x32x16_f16 (layouts in kern_mfma.hip)
-// with K and V as the cache holds them and q and the probabilities as two
-// f16 (hi + lo, 22 bits) after an exact scaling by a power of two (q's row
-// maximum to 2^14 .. 2^15, probabilities by 2^14, so that lo never runs out
-// of exponents); scores, exponentials and sums are f32:
-//   scores: A = K (keys), B = q, k over the dims, so lane (r, h) gets query
-//           r's scores of keys 8 (i/4) + 4 h + i%4 in register i;
-//   output: A = V^T (row a of tile dt = dim ND a + dt), B = the
-//           probabilities, registers 8 s .. 8 s + 7 being step s's keys as
-//           they lie.
-// A tile that holds an infinite or NaN key or value, also one past a query's
-// position (zero probability times infinity), leaves a result that is not
-// finite: the wave then repeats its tiles in f32, key by key.
-// Bound: latency (a block's waves take ceil(context / 256) tiles each).
-// Measured on the config-5 attention (16 heads x 128), k_attn_part +
-// k_attn_combine before: 500 tokens 117 + 14 -> 22 us, 37 tokens 7 + 5 ->
-// 11 us.  The f32 matrix instruction (v_mfma_f32_32x32x2_f32, an eighth of
-// the rate) in both products took 42 and 19 us; the logits' error against
-// float64 is the same either way and as before (3.7e-5 after 500 tokens,
-// four layers).
-constexpr int kPreWaves = 8;
+// k_attn_part for a prompt: chunk c and head h for four queries at a time
+// (tokens i0 .. i0 + 3 of sequence `seq`), so that a block reads the chunk's K
+// and V rows once for all of them.  Every sum runs in k_attn_part's order on
+// the same operands -- half-row dots of two threads per key, the wave
+// reductions over keys 0-63 and 64-127, KG position groups added in order --
+// so the partials, and with them a prompt's results, are bit for bit those of
+// k_attn_part.  q comes through scalar loads (a wave's 64 keys share it),
+// which leaves the LDS to the scores and the group sums.
+// Bound: VALU issue (2 HD multiply-adds per query and key) and a block's chain
+// of loads and barriers.  16 heads x 128, with the combine, us, k_attn_part
+// against it: 500 tokens 115 / 52, 100 tokens 17 / 13, 128 tokens on 8000
+// cached 693 / 284.  Tiles of 8 and 16 queries: 500 tokens 56 and 71 (fewer
+// blocks, each a longer chain).
+constexpr int kTileQ = 4;
 
-template <int ND>  // hd = 32 ND
-__global__ __launch_bounds__(64 * kPreWaves, 2) void k_attn_prefill(
-    const float *__restrict__ qr, int T, int seq, const int32_t *__restrict__ lens, int H, int KVH,
-    const _Float16 *__restrict__ kc, const _Float16 *__restrict__ vc, int ctx,
-    float *__restrict__ out, _Float16 *__restrict__ x16, _Float16 *__restrict__ xs) {
+template <int HD>
+__global__ __launch_bounds__(256) void k_attn_tile(const float *__restrict__ qr, int T, int seq,
+                                                   const int32_t *__restrict__ lens, int H, int KVH,
+                                                   const _Float16 *__restrict__ kc,
+                                                   const _Float16 *__restrict__ vc, int ctx,
+                                                   int chunks, float *__restrict__ part) {
     typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-    typedef _Float16 hv __attribute__((ext_vector_type(ND)));
     typedef float f4 __attribute__((ext_vector_type(4)));
-    typedef float f16v __attribute__((ext_vector_type(16)));
-    constexpr int HD = 32 * ND, NS = HD / 16, ROW = HD + 4;
-    __shared__ __attribute__((aligned(16))) float s_o[kPreWaves][32][ROW];
-    __shared__ float s_m[kPreWaves][32], s_l[kPreWaves][32];
-    const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int head = blockIdx.y, kvh = head / (H / KVH);
-    // the last queries see the most keys: they go first
-    const int i0 = 32 * ((int)gridDim.x - 1 - (int)blockIdx.x);
-    const int base = lens[seq];                            // cached before this call
-    const int qi = min(i0 + r, T - 1), limit = base + qi;  // query r's token and last key
-    const int nkey = base + min(i0 + 32, T), ntile = (nkey + 31) / 32;
-    const int64_t pstride = (int64_t)KVH * HD;
-    const float *qrow = qr + (int64_t)qi * H * HD + head * HD;
-    const _Float16 *kb = kc + (int64_t)seq * ctx * pstride + kvh * HD;
-    const _Float16 *vb = vc + (int64_t)seq * ctx * pstride + kvh * HD;
-    const float root = sqrtf((float)HD);
-    // key of register i in this lane's half
-    const auto key_of = [&](int i) { return 8 * (i >> 2) + 4 * h + (i & 3); };
-    h8 kv[NS];
-    hv vv[16];
-    // tile kt's rows (clamped to the last key: such keys are masked)
-    const auto load_k = [&](int kt) {
-        const _Float16 *kr = kb + min(32 * kt + r, nkey - 1) * pstride + 8 * h;
-#pragma unroll
-        for (int j = 0; j < NS; j++) kv[j] = *reinterpret_cast<const h8 *>(kr + 16 * j);
+    constexpr int HD2 = HD / 2, NK = HD2 / 8, DG = HD / 8, KG = 256 / DG, NV = kAttnChunk / KG;
+    __shared__ float s_dot[2][kTileQ][kAttnChunk];  // half-row dots; [0] then the probabilities
+    __shared__ __attribute__((aligned(16))) float s_o[2][KG * HD];
+    const int h = blockIdx.y, c = blockIdx.z, t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int kvh = h / (H / KVH), i0 = kTileQ * blockIdx.x, nq = min(kTileQ, T - i0);
+    const int base = lens[seq], p0 = c * kAttnChunk;  // cached before this call; chunk start
+    // positions of the chunk that query j of the tile sees (below 1: none)
+    const auto visible = [&](int j) { return min(kAttnChunk, base + i0 + j + 1 - p0); };
+    const auto row = [&](int j) {
+        return part + (((int64_t)(i0 + j) * H + h) * chunks + c) * (HD + 2);
     };
-    const auto load_v = [&](int kt) {
-#pragma unroll
-        for (int i = 0; i < 16; i++)
-            vv[i] = *reinterpret_cast<const hv *>(vb + min(32 * kt + key_of(i), nkey - 1) * pstride +
-                                                  ND * r);
-    };
-    if (wave < ntile) load_k(wave);
-    // q, dims 16 j + 8 h .. + 7 of query r, scaled: hi and lo halves
-    h8 qh[NS], ql[NS];
-    float qscale;  // takes the scores back
-    {
-        f4 qv[2 * NS];
-#pragma unroll
-        for (int j = 0; j < NS; j++) {
-            const f4 *qp = reinterpret_cast<const f4 *>(qrow + 16 * j + 8 * h);
-            qv[2 * j] = qp[0];
-            qv[2 * j + 1] = qp[1];
+    const int most = visible(nq - 1);
+    if (most < 1) {  // the combine skips the chunk by m and l
+        if (t < nq) {
+            row(t)[HD] = -INFINITY;
+            row(t)[HD + 1] = 0.0f;
         }
-        float mx = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 2 * NS; j++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) mx = fmaxf(mx, fabsf(qv[j][e]));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const int ex = 141 - (int)(__float_as_uint(mx) >> 23);  // mx -> [2^14, 2^15)
-        qscale = __builtin_amdgcn_ldexpf(1.0f, -ex);
-#pragma unroll
-        for (int j = 0; j < NS; j++)
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const float v = __builtin_amdgcn_ldexpf(qv[2 * j + (e >> 2)][e & 3], ex);
-                qh[j][e] = (_Float16)v;
-                ql[j][e] = (_Float16)(v - (float)qh[j][e]);
-            }
+        return;
     }
-    f16v O[ND];
-    float m, l;
-    const auto clear = [&] {
+    const int64_t pstride = (int64_t)KVH * HD;  // elements between positions
+    // rows past `most` re-read the last one, never used
+    const int key = t & (kAttnChunk - 1), hf = wave >> 1;
+    const int dg = t % DG, kg = t / DG;
+    h8 kv[NK], vv[NV];
+    {
+        const _Float16 *kr = kc + ((int64_t)seq * ctx + p0 + min(key, most - 1)) * pstride +
+                             kvh * HD + hf * HD2;
+        const _Float16 *vr = vc + ((int64_t)seq * ctx + p0) * pstride + kvh * HD + 8 * dg;
 #pragma unroll
-        for (int dt = 0; dt < ND; dt++) O[dt] = f16v{};
-        m = -INFINITY;
-        l = 0.0f;
-    };
-    // scores of a tile -> probabilities, in place; the running maximum moves
-    // on and the sums so far are scaled to it
-    const auto soften = [&](f16v &S, int kt) {
-        float mt = -INFINITY;
+        for (int u = 0; u < NK; u++) kv[u] = *reinterpret_cast<const h8 *>(kr + 8 * u);
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            S[i] = 32 * kt + key_of(i) <= limit ? S[i] / root : -INFINITY;
-            mt = fmaxf(mt, S[i]);
+        for (int u = 0; u < NV; u++)
+            vv[u] = *reinterpret_cast<const h8 *>(vr + min(kg + u * KG, most - 1) * pstride);
+    }
+    const float *q0 = qr + ((int64_t)i0 * H + h) * HD + hf * HD2;
+    float dot[kTileQ] = {};
+#pragma unroll
+    for (int u = 0; u < NK; u++)
+#pragma unroll
+        for (int s = 0; s < kTileQ; s++) {  // queries past the last repeat it
+            const float *q = q0 + (int64_t)min(s, nq - 1) * H * HD + 8 * u;
+#pragma unroll
+            for (int e = 0; e < 8; e++) dot[s] = __builtin_fmaf(q[e], (float)kv[u][e], dot[s]);
         }
-        const float mn = fmaxf(m, fmaxf(mt, __shfl_xor(mt, 32, 64)));
-        const float alpha = m == mn ? 1.0f : expf(m - mn);
-        m = mn;
-        float ps = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            S[i] = S[i] == -INFINITY ? 0.0f : expf(S[i] - mn);
-            ps += S[i];
+    for (int s = 0; s < kTileQ; s++) s_dot[hf][s][key] = dot[s];
+    __syncthreads();
+    {  // wave j: query j's maximum, probabilities and their sum
+        static_assert(kTileQ == 4, "a wave per query");
+        const float root = sqrtf((float)HD);
+        const int j = wave, np = visible(j);
+        float sc[2], p[2];
+#pragma unroll
+        for (int x = 0; x < 2; x++) {
+            const int k = 64 * x + lane;
+            sc[x] = k < np ? (s_dot[0][j][k] + s_dot[1][j][k]) / root : -INFINITY;
         }
-        l = l * alpha + ps;
+        const float m = fmaxf(wave_max(sc[0]), wave_max(sc[1]));
 #pragma unroll
-        for (int dt = 0; dt < ND; dt++) O[dt] *= alpha;
-    };
-    clear();
-    for (int kt = wave; kt < ntile; kt += kPreWaves) {
-        load_v(kt);  // arrives behind the scores
-        f16v S = f16v{};
-#pragma unroll
-        for (int j = 0; j < NS; j++) S = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[j], ql[j], S, 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < NS; j++) S = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[j], qh[j], S, 0, 0, 0);
-        load_k(min(kt + kPreWaves, ntile - 1));
-#pragma unroll
-        for (int i = 0; i < 16; i++) S[i] *= qscale;
-        soften(S, kt);
+        for (int x = 0; x < 2; x++) {
+            p[x] = 64 * x + lane < np ? expf(sc[x] - m) : 0.0f;
+            s_dot[0][j][64 * x + lane] = p[x];
+        }
+        const float l0 = wave_sum(p[0]), l1 = wave_sum(p[1]);
+        if (lane == 0 && j < nq) {
+            row(j)[HD] = m;
+            row(j)[HD + 1] = l0 + l1;
+        }
+    }
+    __syncthreads();
+    // weighted sums of v, two queries at a time: thread (position group kg,
+    // dims 8 dg .. 8 dg + 7), then the KG groups added in LDS
+#pragma unroll 1
+    for (int j = 0; j < nq; j += 2) {
 #pragma unroll
         for (int s = 0; s < 2; s++) {
-            h8 ph, pl;
+            const int np = visible(j + s);
+            float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const float v = S[8 * s + e] * 16384.0f;
-                ph[e] = (_Float16)v;
-                pl[e] = (_Float16)(v - (float)ph[e]);
-            }
+            for (int u = 0; u < NV; u++)
+                if (kg + u * KG < np) {
+                    const float pk = s_dot[0][j + s][kg + u * KG];
 #pragma unroll
-            for (int dt = 0; dt < ND; dt++) {
-                h8 a;
-#pragma unroll
-                for (int e = 0; e < 8; e++) a[e] = vv[8 * s + e][dt];
-                O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl, O[dt], 0, 0, 0);
-                O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph, O[dt], 0, 0, 0);
-            }
-        }
-    }
-    bool bad = !(l < INFINITY);
-#pragma unroll
-    for (int dt = 0; dt < ND; dt++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            O[dt][i] *= 1.0f / 16384.0f;
-            bad |= !(fabsf(O[dt][i]) < INFINITY);
-        }
-    if (__ballot(bad)) {
-        clear();
-        float *sp = &s_o[wave][0][0];  // this wave's probabilities, [key][query]
-        for (int kt = wave; kt < ntile; kt += kPreWaves) {
-            f16v S = f16v{};
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const _Float16 *kr = kb + min(32 * kt + key_of(i), nkey - 1) * pstride;
-#pragma unroll 1
-                for (int d = 0; d < HD; d++) S[i] = __builtin_fmaf(qrow[d], (float)kr[d], S[i]);
-            }
-            soften(S, kt);
-#pragma unroll
-            for (int i = 0; i < 16; i++) sp[key_of(i) * ROW + r] = S[i];
-            chain_detail::wave_lds_sync();
-#pragma unroll 1
-            for (int k = 0; k < 32; k++) {
-                const int key = 32 * kt + k;
-                if (key > limit) continue;
-                const float pk = sp[k * ROW + r];
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const hv vk = *reinterpret_cast<const hv *>(vb + key * pstride + ND * key_of(i));
-#pragma unroll
-                    for (int dt = 0; dt < ND; dt++)
-                        O[dt][i] = __builtin_fmaf(pk, (float)vk[dt], O[dt][i]);
+                    for (int e = 0; e < 8; e++) acc[e] = __builtin_fmaf(pk, (float)vv[u][e], acc[e]);
                 }
-            }
-            chain_detail::wave_lds_sync();
+            f4 *o = reinterpret_cast<f4 *>(&s_o[s][kg * HD + 8 * dg]);
+            o[0] = f4{acc[0], acc[1], acc[2], acc[3]};
+            o[1] = f4{acc[4], acc[5], acc[6], acc[7]};
         }
-    }
-    l += __shfl_xor(l, 32, 64);
-    if (h == 0) {
-        s_m[wave][r] = m;
-        s_l[wave][r] = l;
-    }
+        __syncthreads();
+        if (t < 2 * HD && j + t / HD < nq) {
+            const int s = t / HD, d = t % HD;
+            float o = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {  // dims ND key_of(i) .. + ND - 1
-        typedef float fv __attribute__((ext_vector_type(ND)));
-        fv v;
-#pragma unroll
-        for (int dt = 0; dt < ND; dt++) v[dt] = O[dt][i];
-        *reinterpret_cast<fv *>(&s_o[wave][r][ND * key_of(i)]) = v;
-    }
-    __syncthreads();
-    // merge: 16 threads per query, HD / 16 dims each; the row also stays in
-    // s_o[0] for the output projection's pieces
-    const int qq = tid >> 4, d0 = (tid & 15) * (HD / 16);
-    float M = -INFINITY, den = 0.0f;
-#pragma unroll
-    for (int w = 0; w < kPreWaves; w++) M = fmaxf(M, s_m[w][qq]);
-    float acc[HD / 16];
-#pragma unroll
-    for (int e = 0; e < HD / 16; e++) acc[e] = 0.0f;
-#pragma unroll
-    for (int w = 0; w < kPreWaves; w++) {
-        const float mw = s_m[w][qq];
-        if (mw != -INFINITY) {
-            const float f = expf(mw - M);
-            den += f * s_l[w][qq];
-#pragma unroll
-            for (int e = 0; e < HD / 16; e++) acc[e] += f * s_o[w][qq][d0 + e];
+            for (int g = 0; g < KG; g++) o += s_o[s][g * HD + d];
+            row(j + s)[d] = o;
         }
+        __syncthreads();
     }
-#pragma unroll
-    for (int e = 0; e < HD / 16; e++) {
-        const float v = acc[e] / den;
-        s_o[0][qq][d0 + e] = v;
-        if (i0 + qq < T) out[(int64_t)(i0 + qq) * H * HD + head * HD + d0 + e] = v;
-    }
-    if (!x16) return;
-    __syncthreads();
-    if (tid < 32 * ND && i0 + tid / ND < T)
-        act16_subblock(&s_o[0][tid / ND][32 * (tid % ND)], i0 + tid / ND, H * HD,
-                       head * ND + tid % ND, x16, xs);
 }
 
 // f32::total_cmp order as a signed integer key
@@ -821,16 +707,13 @@ hipError_t launch_attention(const float *qr, int nq, int T, int seq0, const int3
                             _Float16 *xs) {
     if (nq <= 0) return hipSuccess;
     if (x16 && ((H * hd) % 256 || hd % 32 || hd > 256)) return hipErrorInvalidValue;
-    if (nq == T && T >= kPrefillMin && (hd == 32 || hd == 64 || hd == 128)) {  // one sequence
-        const dim3 pg((T + 31) / 32, H), pb(64 * kPreWaves);
-        auto *kern = hd == 32 ? k_attn_prefill<1> : hd == 64 ? k_attn_prefill<2> : k_attn_prefill<4>;
-        hipLaunchKernelGGL(kern, pg, pb, 0, st, qr, T, seq0, lens, H, KVH, kc, vc, ctx, out, x16,
-                           xs);
-        return hipGetLastError();
-    }
     const int chunks = (ctx + kAttnChunk - 1) / kAttnChunk;
     const dim3 grid(nq, H, chunks);
-    if (hd <= 64)
+    if (nq == T && T >= kTileMin && (hd == 32 || hd == 64 || hd == 128)) {  // one sequence
+        auto *kern = hd == 32 ? k_attn_tile<32> : hd == 64 ? k_attn_tile<64> : k_attn_tile<128>;
+        hipLaunchKernelGGL(kern, dim3((T + kTileQ - 1) / kTileQ, H, chunks), dim3(256), 0, st, qr,
+                           T, seq0, lens, H, KVH, kc, vc, ctx, chunks, part);
+    } else if (hd <= 64)
         hipLaunchKernelGGL(k_attn_part<4>, grid, dim3(256), 0, st, qr, nq, T, seq0, lens, H, KVH,
                            hd, kc, vc, ctx, chunks, part);
     else if (hd <= 128)

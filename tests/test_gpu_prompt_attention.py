@@ -1,5 +1,6 @@
-"""The prompt attention kernel (one sequence of 16 or more tokens, head_dim
-32, 64 or 128) through the decoder model, against the oracle's engine."""
+"""The prompt attention kernel (several tokens of one sequence, head_dim 32,
+64 or 128) through the decoder model: against the oracle's engine, and bit
+for bit against the kernel of single tokens."""
 import numpy as np
 import pytest
 
@@ -19,8 +20,8 @@ def _model_config(hd, H, KVH, qt):
                                     L.TYPE_Q8_0), attn_type=qt)
 
 
-# T around the 32-key tiles, past the eight waves' first tiles (256 keys),
-# and below the kernel's range; then a second prompt on a filled cache
+# T below the kernel's fewest tokens, above them, and past two 128-position
+# chunks; then a second prompt on a filled cache
 @pytest.mark.parametrize("T", [15, 16, 31, 32, 33, 65, 290])
 @pytest.mark.parametrize("hd,H,KVH,qt", [(32, 4, 2, L.TYPE_Q8_0), (64, 4, 4, L.TYPE_Q4_K),
                                          (128, 2, 1, L.TYPE_Q4_K)])
@@ -32,6 +33,31 @@ def test_prompt_attention_matches_oracle(hd, H, KVH, qt, T):
         for c in ([(7 * i + 3) % 64 for i in range(T)], [(5 * i + 1) % 64 for i in range(37)], [9]):
             g = m.forward(np.array([c]))[0]
             assert rel(g, ref.forward(c).astype(np.float64)) < LOGIT_TOL
+
+
+# T and the cached tokens before it around the kernel's fewest tokens, its
+# 4-query tiles and the 128-position chunks
+@pytest.mark.parametrize("cached", [0, 1, 100, 128])
+@pytest.mark.parametrize("T", [2, 39, 40, 41, 42, 43, 64, 127, 128, 129, 200, 273])
+@pytest.mark.parametrize("hd,H,KVH", [(32, 8, 2), (64, 4, 4), (128, 2, 1)])
+def test_prompt_attention_is_the_one_token_kernel(hd, H, KVH, T, cached):
+    """A prompt's logits have the bits of the same prompt with its last token
+    in a call of its own: attention runs every sum in one order (the Q8_0
+    products and experts of the decoder take each token alone anyway)."""
+    mc = _model_config(hd, H, KVH, L.TYPE_Q8_0)
+    w = synth_model(mc, seed=hd)
+    tok = np.random.default_rng(T + cached).integers(0, 64, (1, cached + T)).astype(np.int32)
+    with L.Model(mc.desc(1, 300, 420, E.ROPE_ABSOLUTE), w) as m:
+        out = []
+        for cut in (cached + T, cached + T - 1):
+            m.reset()
+            if cached:
+                m.forward(tok[:, :cached])
+            if cut > cached:
+                out.append(m.forward(tok[:, cached:cut])[0])
+            if cut < cached + T:
+                out[-1] = m.forward(tok[:, cut:])[0]
+    assert np.array_equal(out[0], out[1])
 
 
 @pytest.mark.parametrize("sign", [1.0, -1.0])
