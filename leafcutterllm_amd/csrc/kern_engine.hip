@@ -359,6 +359,9 @@ __global__ __launch_bounds__(256) void k_attn_part(const float *__restrict__ qr,
 }
 
 // out[q][h*hd + d] = sum_c e^(m_c - M) o_c[d] / sum_c e^(m_c - M) l_c
+// over the chunks with a visible position (else m = -inf and l = 0).  One whose
+// scores are all NaN has m = -inf too (a maximum passes NaN over) but l = NaN:
+// it counts, and the result is NaN as the softmax's is.
 // With x16, the block's hd outputs also go to the matrix-core activation
 // format (act16_subblock over the row of H * hd, staged through LDS).
 __global__ __launch_bounds__(256) void k_attn_combine(const float *__restrict__ part, int nq,
@@ -375,7 +378,8 @@ __global__ __launch_bounds__(256) void k_attn_combine(const float *__restrict__ 
     float den = 0.0f;
     for (int c = 0; c < chunks; c++) {
         const float mc = pp[c * (hd + 2) + hd];
-        if (mc != -INFINITY) den += expf(mc - M) * pp[c * (hd + 2) + hd + 1];
+        const float lc = pp[c * (hd + 2) + hd + 1];
+        if (mc != -INFINITY || lc != 0.0f) den += expf(mc - M) * lc;
     }
     for (int d = threadIdx.x; d < hd; d += blockDim.x) {
         float acc = 0.0f;

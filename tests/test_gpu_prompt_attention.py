@@ -85,3 +85,25 @@ def test_infinite_value_stays_with_its_readers(sign):
     for a, b in zip(*seen):
         assert np.array_equal(a["topk_idx"], b["topk_idx"][:T - 1])
         np.testing.assert_allclose(b["topk_w"][:T - 1], a["topk_w"], rtol=1e-4)
+
+
+@pytest.mark.parametrize("cut", [0, 128])
+def test_nan_score_alone_in_its_chunk(cut):
+    """A token whose own key scores NaN (K past f16's range with contributions
+    of both signs) at position 128, the only one its query sees in that
+    128-position chunk: its logits are not finite, in a prompt and in a call
+    of one token."""
+    mc = _model_config(64, 4, 4, L.TYPE_F32)
+    w = synth_model(mc, seed=4)
+    d, A, j, T = 256, 63, 17, 129
+    embd = w["token_embd"].view(np.float32).reshape(64, d)
+    embd[A] = 0
+    embd[A, j] = 1.0
+    for lw in w["layers"]:
+        lw["attn_norm"][j] = 100.0
+        lw["attn_k"].view(np.float32).reshape(-1, d)[:, j] = 100.0  # 16 * 100 * 100 past 65504
+    tok = np.array([[(7 * i + 3) % 61 for i in range(T - 1)] + [A]])
+    with L.Model(mc.desc(1, 160, 160, E.ROPE_ABSOLUTE), w) as m:
+        if cut:
+            assert np.all(np.isfinite(m.forward(tok[:, :cut])))
+        assert not np.any(np.isfinite(m.forward(tok[:, cut:])))
