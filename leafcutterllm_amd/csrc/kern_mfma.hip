@@ -485,14 +485,17 @@ __device__ __forceinline__ void block_pass(g_u8 *const (&wb)[MATS], uint32_t lo,
 // scale) a super-block starts with
 //   acc = acc * (d' / d) - (dmin / d) * sum_j m_j V_j
 // and its products sc*q are added to acc by the MFMAs themselves; the result
-// is acc * d of the last super-block.  The rescaling rounds once per
-// super-block and element, as the fma it replaces did.  A super-block with
-// d = 0 keeps d' and decodes with zero scales.
+// is acc * d of the last super-block.  A super-block with d = 0 keeps d' and
+// decodes with zero scales.  Rounding, all in f32: the MFMAs add to the whole
+// running total (a 32-token pass starts each super-block's S from zero), and
+// per super-block 1 / d, d' / d, dmin / d, its product with the min sum and
+// the fma round once each (the split layout: d' / d and the total twice).
+// With H exact in f16 the down product's error against float64 is 2.3e-7 to
+// 2.7e-7 of the result at F = 512 to 14336 where 32-token passes leave 1.1e-7
+// to 1.4e-7; the layer's, 3.6e-4 from its f16 activations, is the same.
 // Bound: VALU issue beside the MFMAs, and the activation loads.  Per
 // super-block and wave (gate/up) 68 MFMAs against ~530 VALU instructions for
-// 64 tokens, where two 32-token passes issue 68 against ~850; the matrix
-// cores are busy 40% of the launch (26% before).  Without the decode the
-// launch would take 540 of 620 us, without the activation loads 533.
+// 64 tokens, where two 32-token passes issue 68 against ~850.
 // Measured (gate/up + down, us, 32-token passes before): config 2 T = 1000
 // 756 + 392 -> 621 + 371, T = 300 286 + 137 -> 264 + 137; config 3 T = 1801
 // 303 + 174 -> 262 + 156, T = 700 149 + 85 -> 138 + 88.
@@ -534,12 +537,14 @@ __device__ __forceinline__ void wide_store_sums(uint8_t *stage, u32x2 v, int wav
     *reinterpret_cast<u32x2 *>(stage + kSumsOffW + wave * 512 + 8 * lane) = v;
 }
 
-// The scale `d` of the coming super-block for accumulators in units of
-// `unit`: d, or `unit` itself when d is zero.  rd = 1 / (the new unit).
-__device__ __forceinline__ float next_unit(float d, float unit, float &rd) {
+// Accumulators in units of `unit` go over to the coming super-block's scale
+// d, or keep their unit when d is zero: *= ratio (1 where the unit stays the
+// same, else the rounded quotient), rd = 1 / (the new unit).
+__device__ __forceinline__ void next_unit(float d, float &unit, float &ratio, float &rd) {
     const float u = d != 0.0f ? d : unit;
     rd = 1.0f / u;
-    return u;
+    ratio = u == unit ? 1.0f : unit * rd;
+    unit = u;
 }
 
 // acc = acc * ratio + t * (sum_j m_j V_j) for NT token tiles
@@ -579,13 +584,12 @@ __device__ __forceinline__ void step_wide(g_u8 *const (&wb)[MATS], uint32_t lo,
         hd[m] = SPLIT ? unpack_hdr_split(w[m].hdr, w[m].db) : unpack_hdr16(w[m].hdr);
         w[m].hdr = load_hdr<SPLIT>(wb[m], lo, kn);
         w[m].db = load_db<SPLIT>(wb[m], dbo[m], kn);
-        float rd;
-        const float u = next_unit(hd[m].d, unit[m], rd);
+        float ratio, rd;
+        next_unit(hd[m].d, unit[m], ratio, rd);
         const half8 mo = min_operand(hd[m], h);
         // lanes of half h hold the mins of sub-blocks 4h .. 4h + 3
-        rescale<NT>(acc[m], unit[m] * rd, -hd[m].dmin * rd, amin, SPLIT ? mo * k0 : mo);
+        rescale<NT>(acc[m], ratio, -hd[m].dmin * rd, amin, SPLIT ? mo * k0 : mo);
         if (SPLIT) rescale<NT>(acc[m], 1.0f, -hd[m].dmin2 * rd, amin, mo * k1);
-        unit[m] = u;
         // d = 0 (d2 in the split layout's second half): zero scales
         hd[m].sc03 = hd[m].d != 0.0f ? hd[m].sc03 : 0;
         hd[m].sc47 = (SPLIT ? hd[m].d2 : hd[m].d) != 0.0f ? hd[m].sc47 : 0;
@@ -600,12 +604,10 @@ __device__ __forceinline__ void step_wide(g_u8 *const (&wb)[MATS], uint32_t lo,
         if (SPLIT && u == 4) {  // sub-blocks 4-7: their own d
 #pragma unroll
             for (int m = 0; m < MATS; m++) {
-                float rd;
-                const float un = next_unit(hd[m].d2, unit[m], rd);
-                const float ratio = unit[m] * rd;
+                float ratio, rd;
+                next_unit(hd[m].d2, unit[m], ratio, rd);
 #pragma unroll
                 for (int j = 0; j < NT; j++) acc[m][j] *= ratio;
-                unit[m] = un;
             }
         }
         if (NT == 2 && u == 4) {
