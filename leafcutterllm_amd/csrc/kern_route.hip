@@ -1460,10 +1460,12 @@ __global__ __launch_bounds__(64 * kSigWaves) void k_route_sig(RouterArgs a, Chai
     // streams, one for each of its FBW waves.  Those are tiles of 32 experts:
     // every lane of a wave reads its LDS rows whether it owns a chain or not,
     // so a tile of 32 takes little longer than one of 8, and the block's four
-    // waves go over 256 experts twice instead of eight times (config 4's layer
-    // at one uncertified token 362 -> 200 us; certified tokens 79 -> 80).
-    // The LDS (139 KB) leaves one block per CU; one token needs at most 128.
-    constexpr int kFbCols = 128, kFbExperts = 32;
+    // waves go over 256 experts twice instead of eight times.  Chunks of 64
+    // columns, two ahead, keep the kernel at two waves per SIMD and 74 KB of
+    // LDS, as it is without the fallback (chunks of 128: one, 140 KB).  Config
+    // 4's layer, tiles of 8 / of 32 in chunks of 64 / of 128, us: uncertified
+    // tokens 360 / 201 / 198, certified ones 78.4 / 78.5 / 79.1.
+    constexpr int kFbCols = 64, kFbExperts = 32;
     constexpr int kChainFloats = chain_lds_floats(1 + 8, 256);
     constexpr int kFbFloats = chain_lds_floats(1 + kFbExperts, kFbCols);
     constexpr int kFbAll = FBW > 1 ? kFbFloats * FBW : 0;
