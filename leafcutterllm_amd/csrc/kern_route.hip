@@ -377,7 +377,7 @@ __device__ void dispatch_block(const RouterArgs &a, int (*s_cw)[kMaxE], int *s_o
     }
 }
 
-// The same dispatch of at most 64 GMAX assignments by one wave, without the
+// The same dispatch of at most 64 kDispGroups assignments by one wave, without the
 // block's barriers and LDS counters: assignment 64 g + l sits in lane l, the
 // ballots of its expert's eight bits give every lane both its own matches
 // (rank) and, reading the lane number as an expert, that expert's count.
@@ -1687,7 +1687,10 @@ bool route_fast_ok(const RouterArgs &a) {
 // cost ~2 us.  Config 5's router, one block against the split (with the
 // norm's 512-thread form and the one-wave dispatch on both sides of the
 // second figure): T = 16 30 -> 16 us, T = 9 32 -> 16, T = 37 31 -> 20.
-// E <= 8 (one expert per wave) has nothing to share.
+// E <= 8 (one expert per wave) has nothing to share, and layers of 9 to 31
+// experts have no buffers to share through (lcmoe_create allocates them from
+// kParallelBoundsMinE on, for the one-token router): their bounds are two to
+// four rounds of a block's eight waves.
 // Returns the logarithm.
 static int fast_split(const RouterArgs &a) {
     int l = 0;

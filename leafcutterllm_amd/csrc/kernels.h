@@ -44,12 +44,17 @@ struct RouterArgs {
     const float *xin = nullptr, *norm_w = nullptr;
     float norm_eps = 0.0f;
     float *xn = nullptr;
-    // Certified sigmoid-group router: float64 logit and bound per (t, e),
-    // per-token block counters, and per-token fallback marks (1: the exact
-    // chains decide this token); the chain and select launches that follow
-    // it serve only the marked tokens when `flag` is set.
-    uint64_t *bnd = nullptr;    // [T, E, 2]: keys (klo, khi), (km, finite) as float pairs
+    // Certified routers whose blocks share a token: what the bound blocks
+    // publish per (t, e) and the per-token counters of finished blocks.  The
+    // parallel-bounds router (launch_route_sig) stores the certification keys
+    // (klo, khi), (km, finite) as float pairs; the fast router the float64
+    // logit sum and its error bound.  Null: the fast router keeps one block
+    // per token.
+    uint64_t *bnd = nullptr;    // [T, E, 2]
     uint32_t *tsync = nullptr;  // [T] zero-initialised
+    // Parallel-bounds router: per-token fallback marks (1: the exact chains
+    // decide this token); the chain and select launches that follow it serve
+    // only the marked tokens when `flag` is set.
     int32_t *flag = nullptr;    // [T]
 };
 // The exact router: logits, limbs, top-k, dispatch.

@@ -1,6 +1,6 @@
-// CpuBackend::rms_norm, bit for bit, as a per-wave device function shared by
-// the stand-alone norm kernel (kern_generic.hip) and the router entry kernel
-// that fuses it (kern_route.hip).
+// CpuBackend::rms_norm, bit for bit: the stand-alone norm on a block or a wave
+// (kern_generic.hip), and the chains and roundings that the router's entry
+// runs on a row it keeps in LDS (stage_row in kern_route.hip).
 #pragma once
 
 #include "device_common.h"
@@ -84,7 +84,6 @@ __device__ __forceinline__ float chain_sum(const float4 *c, int n16, float acc) 
 // LDS floats rmsnorm_wave<CHUNK> needs
 template <int CHUNK = kNormChunk>
 constexpr int rmsnorm_lds() { return 4 * (CHUNK / 4 + 4); }
-constexpr int kRmsnormLds = rmsnorm_lds<>();
 
 // LDS stores of the wave visible to its own later reads
 __device__ __forceinline__ void wave_lds_sync() {
@@ -244,7 +243,6 @@ __device__ __attribute__((always_inline)) inline void rmsnorm_block(const float 
 
 }  // namespace rmsnorm_detail
 
-using rmsnorm_detail::kRmsnormLds;
 using rmsnorm_detail::rmsnorm_lds;
 using rmsnorm_detail::rmsnorm_wave;
 using rmsnorm_detail::rmsnorm_block;
